@@ -327,18 +327,13 @@ int ipc_ctx_kernel_times(ipc_ctx* ctx, double* total_ms, long long* calls);
 #define IPC_MLP_OUT 3
 #define IPC_MLP_PARAMS 144899
 /* Forward pass. work (float [6 * 256 * n]) keeps Z1, H1, Z2, H2, Z3, H3 for
- * a backward pass; with work = NULL, scratch (float [3 * 256 * n]) holds the
- * activations. */
+ * a backward pass; with work = NULL, scratch must be given (float
+ * [3 * 256 * n]; the activations stay on the chip and it is left untouched). */
 int ipc_mlp_forward(const float* params, int n, const float* x, float* y, float* work, float* scratch, void* stream);
-/* Inference that allocates nothing: ipc_mlp_forward with work = NULL, its
- * activations held in a device array inside the library (3 * 256 *
- * IPC_MLP_NOALLOC_MAX_ROWS floats, 12 MiB, one per GPU the library runs on,
- * kept until the process ends) instead of a scratch argument. No
+/* Inference without a scratch argument: ipc_mlp_forward with work = NULL. No
  * counterpart in the reference: it is for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops). n must not exceed
- * IPC_MLP_NOALLOC_MAX_ROWS (IPC_EINVAL otherwise). Every call on one GPU
- * shares that array, so calls that overlap on one GPU (other streams,
- * other threads) race; calls on one stream are ordered and safe. */
+ * IPC_MLP_NOALLOC_MAX_ROWS (IPC_EINVAL otherwise). Calls share nothing. */
 #define IPC_MLP_NOALLOC_MAX_ROWS 4096
 int ipc_mlp_forward_noalloc(const float* params, int n, const float* x, float* y, void* stream);
 /* Backward pass of the forward pass that filled `work`: ADDS the gradient of

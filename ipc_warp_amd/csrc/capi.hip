@@ -228,7 +228,7 @@ int ipc_mlp_forward(const float* params, int n, const float* x, float* y, float*
   if (n == 0) return IPC_OK;
   if (!params || !x || !y || (!work && !scratch)) return fail(IPC_EINVAL, "mlp_forward: null pointer");
   if ((long long)n * IPC_MLP_HIDDEN * 6 > (1ll << 31)) return fail(IPC_EINVAL, "mlp_forward: batch too large");
-  return hip_status(ipcd::mlp_forward(params, n, x, y, work, scratch, static_cast<hipStream_t>(stream)),
+  return hip_status(ipcd::mlp_forward(params, n, x, y, work, static_cast<hipStream_t>(stream)),
                     "mlp_forward");
 }
 
@@ -237,7 +237,7 @@ int ipc_mlp_forward_noalloc(const float* params, int n, const float* x, float* y
   if (n > IPC_MLP_NOALLOC_MAX_ROWS) return fail(IPC_EINVAL, "mlp_forward_noalloc: n exceeds IPC_MLP_NOALLOC_MAX_ROWS");
   if (n == 0) return IPC_OK;
   if (!params || !x || !y) return fail(IPC_EINVAL, "mlp_forward_noalloc: null pointer");
-  return hip_status(ipcd::mlp_forward_noalloc(params, n, x, y, static_cast<hipStream_t>(stream)),
+  return hip_status(ipcd::mlp_forward(params, n, x, y, nullptr, static_cast<hipStream_t>(stream)),
                     "mlp_forward_noalloc");
 }
 

@@ -1,24 +1,16 @@
 // Learned warm start: the MLP 48 -> 256 -> 256 -> 256 -> 3 (GELU, fp32) that
 // predicts a vertex's converged Newton displacement. Forward, backward, loss
-// and Adam are hand-written kernels; one tiled GEMM kernel with fused
-// epilogues covers every layer product.
+// and Adam are hand-written kernels: one launch for the four layers, two for
+// the backward pass, every layer product on the fp32 matrix instructions.
 //
 // Parameters are one flat fp32 array: W1 [256][48], b1 [256], W2 [256][256],
 // b2, W3 [256][256], b3, W4 [3][256], b4 [3] (W row-major, out x in).
 // Activations of a forward pass with backward in mind ("work") hold
 // Z1, H1, Z2, H2, Z3, H3, each [n][256] (pre-activation and GELU output).
 #include <cmath>
-#include <mutex>
 
 #include "../../include/ipc_warp_amd.h"
 #include "ipc_kernels.hpp"
-
-// Activations of ipc_mlp_forward_noalloc: a file-scope device array (one
-// copy per GPU, held until the process ends) instead of a caller or library
-// buffer, so that inference allocates nothing. Host code must use the
-// address hipGetSymbolAddress returns on each device (scratch_on_device),
-// never this name: on the host it is a stand-in, not a device address.
-static __device__ __align__(256) float scratch[3 * IPC_MLP_HIDDEN * IPC_MLP_NOALLOC_MAX_ROWS];
 
 namespace ipcd {
 
@@ -34,107 +26,552 @@ constexpr long long kOffB4 = kOffW4 + (long long)kOut * kHid;
 constexpr long long kParams = kOffB4 + kOut;
 static_assert(kParams == IPC_MLP_PARAMS, "parameter layout");
 
-__device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
+// Phi(z), the normal distribution function, and E = exp(-z^2 / 2):
+//     Phi(-|z|) = E q(|z|),  q(a) = erfcx(a / sqrt 2) / 2 = t P(t),  t = 1 / (1 + 0.3 a)
+// with P of degree 9 fitted for the least relative error on [0, 14] (3.4e-9;
+// beyond it E underflows). About 25 instructions without a branch; erff and
+// expf took four times as many, as long as the matrix products themselves.
+// In fp32 gelu's error is 4.4e-8 rms (erff: 4.9e-8), its derivative's 3.3e-8
+// (2.6e-8), both over normally distributed z; Phi's lower tail keeps its
+// relative precision.
+__device__ __forceinline__ float phi_cdf(float z, float& e) {
+  const float a = fabsf(z);
+  e = __builtin_amdgcn_exp2f(z * z * -0.72134752044448170f);
+  const float t = __builtin_amdgcn_rcpf(fmaf(0.3f, a, 1.0f));
+  float p = -2.061283588e-02f;
+  p = fmaf(p, t, 1.123758107e-01f);
+  p = fmaf(p, t, -2.280675769e-01f);
+  p = fmaf(p, t, 1.915817857e-01f);
+  p = fmaf(p, t, -7.924740762e-02f);
+  p = fmaf(p, t, 9.605786204e-02f);
+  p = fmaf(p, t, 7.842557132e-02f);
+  p = fmaf(p, t, 1.102273241e-01f);
+  p = fmaf(p, t, 1.195728406e-01f);
+  p = fmaf(p, t, 1.196866333e-01f);
+  const float lo = e * (p * t);
+  return z >= 0.f ? 1.0f - lo : lo;
+}
+__device__ __forceinline__ float gelu(float z) {
+  float e;
+  return z * phi_cdf(z, e);
+}
 __device__ __forceinline__ float gelu_grad(float z) {
   // d/dz [z Phi(z)] = Phi(z) + z phi(z)
-  return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
+  float e;
+  const float c = phi_cdf(z, e);
+  return fmaf(z * 0.39894228040143268f, e, c);
 }
 
-enum Epi { EPI_BIAS = 0, EPI_BIAS_GELU = 1, EPI_GELU_BACK = 2, EPI_ATOMIC = 3 };
+// ------------------------------------------------------------- MFMA tiles ----
+// Every layer product runs on the fp32 matrix instructions (fp32 inputs and
+// accumulators, as the VALU code before them had). Layouts used, for lane l:
+//   16x16x4: A row l % 16, k l / 16; B column l % 16, k l / 16; result
+//            column l % 16, rows 4 (l / 16) + 0..3
+//   32x32x2: A row l % 32, k l / 32; B column l % 32, k l / 32; result
+//            column l % 32, register q row 8 (q / 4) + 4 (l / 32) + q % 4
+using f4 = __attribute__((ext_vector_type(4))) float;
+using f16 = __attribute__((ext_vector_type(16))) float;
+using f2 = __attribute__((ext_vector_type(2))) float;
 
-constexpr int kTile = 64, kTk = 16, kGemmThreads = 256;
+// Wide global accesses at the 4-byte alignment the entry points ask for.
+__device__ __forceinline__ f4 ld4(const float* p) { f4 v; __builtin_memcpy(&v, p, 16); return v; }
+__device__ __forceinline__ f2 ld2(const float* p) { f2 v; __builtin_memcpy(&v, p, 8); return v; }
+__device__ __forceinline__ void st4(float* p, f4 v) { __builtin_memcpy(p, &v, 16); }
+__device__ __forceinline__ void st2(float* p, f2 v) { __builtin_memcpy(p, &v, 8); }
 
-// C[r][c] = epilogue( sum_k A(r, k) B(k, c) ), 64 x 64 tiles, 16-deep K
-// steps staged in LDS, 4 x 4 outputs per thread.
-//   A(r, k) = TA ? A[k * lda + r] : A[r * lda + k]
-//   B(k, c) = TB ? B[c * ldb + k] : B[k * ldb + c]
-// EPI_BIAS:      C = acc + bias[c]
-// EPI_BIAS_GELU: P[r][c] = acc + bias[c]; C = gelu(P)
-// EPI_GELU_BACK: C = acc * gelu'(P[r][c])
-// EPI_ATOMIC:    C += acc (atomically; blockIdx.z splits the K range)
-template <bool TA, bool TB, int EPI>
-__global__ void __launch_bounds__(kGemmThreads) gemm_kernel(int R, int Cn, int K, const float* __restrict__ A, int lda,
-                                                            const float* __restrict__ B, int ldb, float* C, int ldc,
-                                                            const float* __restrict__ bias, float* P, int k_chunk) {
-  __shared__ float As[kTk][kTile + 4];
-  __shared__ float Bs[kTk][kTile + 4];
-  int tr = threadIdx.x / 16, tc = threadIdx.x % 16;
-  int r0 = blockIdx.y * kTile, c0 = blockIdx.x * kTile;
-  int k_begin = blockIdx.z * k_chunk;
-  int k_end = min(K, k_begin + k_chunk);
-  float acc[4][4];
+// The row kernels keep two or three weight stages in registers: two waves a
+// SIMD hold them without a spill.
+#define kFewWaves __attribute__((amdgpu_waves_per_eu(2, 2)))
+constexpr int kThreads = 512;  // 8 waves, 32 of the 256 columns each
+constexpr int kLd = kHid + 4;  // LDS row stride of an activation tile: a column of 16-byte reads meets every bank once
+constexpr int kLdIn = kIn + 4;
+
+// A wave's share of 64 k of a weight matrix, in registers: 32 columns of W^T
+// (wt_) or W (w_). A layer is four of them; the kernels keep up to three, so
+// that the loads of a stage run under the products of the two before it and
+// across the barriers between layers. (With the loads beside their use a
+// workgroup took 22 us for 16 rows, one load latency per stage.) The waves
+// start a layer at different stages: rows of W are 1 KB apart, so in one
+// column of it every wave would ask the same few L2 channels.
+struct Stage {
+  f4 b[8];
+};
+__device__ __forceinline__ int stage_k(int i, int wave) { return 64 * ((i + wave) & 3); }
+
+// acc[rt][t] += A W^T for the wave's columns c0 + 16 t + l % 16: A the
+// workgroup's 16 RT rows in LDS (row stride ld), W [256][K] row-major. A k
+// step of 16 is four matrix instructions whose lane groups take k = 4 (l /
+// 16) + s, so both operands are read 16 bytes at a time.
+template <int K, int Q = 4>
+__device__ __forceinline__ void wt_load(Stage& S, const float* __restrict__ W, int k0, int c0, int l) {
+  const float* w = W + (c0 + (l & 15)) * K + k0 + 4 * (l >> 4);
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int q = 0; q < Q; ++q) {
+    S.b[q] = ld4(w + 16 * q);
+    S.b[4 + q] = ld4(w + 16 * K + 16 * q);
+  }
+  __builtin_amdgcn_sched_barrier(0);  // the loads are issued here, not where they are used
+}
+template <int RT, int Q = 4>
+__device__ __forceinline__ void wt_mul(f4 acc[RT][2], const Stage& S, const float* act, int ld, int k0, int l) {
+  const float* ap = act + (l & 15) * ld + k0 + 4 * (l >> 4);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.f;
-  for (int k0 = k_begin; k0 < k_end; k0 += kTk) {
-    // stage A tile (64 rows x 16 k) and B tile (16 k x 64 cols): 1024 values each, 4 per thread
+  for (int q = 0; q < Q; ++q) {
+    f4 a[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) a[rt] = *reinterpret_cast<const f4*>(ap + 16 * rt * ld + 16 * q);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][s], S.b[4 * t + q][s], acc[rt][t], 0, 0, 0);
+  }
+}
+
+// acc[rt][t] += A W for the wave's columns c0 + 2 (l % 16) + t: W [256][256]
+// row-major, read 8 bytes a lane (16 lanes on 128 consecutive bytes).
+__device__ __forceinline__ void w_load(Stage& S, const float* __restrict__ W, int k0, int c0, int l) {
+  const float* w = W + (k0 + 4 * (l >> 4)) * kHid + c0 + 2 * (l & 15);
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int s = 0; s < 4; s += 2) {
+      const f2 u = ld2(w + (16 * q + s) * kHid), v = ld2(w + (16 * q + s + 1) * kHid);
+      S.b[2 * q + s / 2] = f4{u[0], u[1], v[0], v[1]};
+    }
+  __builtin_amdgcn_sched_barrier(0);
+}
+template <int RT>
+__device__ __forceinline__ void w_mul(f4 acc[RT][2], const Stage& S, const float* act, int k0, int l) {
+  const float* ap = act + (l & 15) * kLd + k0 + 4 * (l >> 4);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    f4 a[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) a[rt] = *reinterpret_cast<const f4*>(ap + 16 * rt * kLd + 16 * q);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][s], S.b[2 * q + s / 2][2 * (s & 1) + t], acc[rt][t],
+                                                            0, 0, 0);
+  }
+}
+
+template <int RT>
+__device__ __forceinline__ void clear(f4 acc[RT][2]) {
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt][0] = acc[rt][1] = f4{0.f, 0.f, 0.f, 0.f};
+}
+
+// rows [r0, r0 + R) of src [n][W] into LDS, zero past n
+template <int R, int W>
+__device__ __forceinline__ void stage_rows(float* dst, int ld, const float* __restrict__ src, long long r0, int n) {
+  constexpr int kQ = W / 4;
+  for (int i = threadIdx.x; i < R * kQ; i += kThreads) {
+    const int row = i / kQ, q = i - row * kQ;
+    const f4 v = r0 + row < n ? ld4(src + (r0 + row) * W + 4 * q) : f4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<f4*>(dst + row * ld + 4 * q) = v;
+  }
+}
+
+// --------------------------------------------------------------- forward ----
+// All four layers of R rows in one workgroup: the activations stay in LDS and
+// the weights (0.58 MB) come from L2. KEEP stores Z and H of each layer. The
+// bound is the CU's own reads of the weights (64 bytes of each of 16 rows an
+// instruction) beside the products: 20 us for up to 4096 rows, where four
+// launches of a VALU product took 120 us; 89 of 148 TFLOP/s at 121,904 rows
+// (17 before).
+template <int R, bool KEEP>
+__device__ __forceinline__ void layer_out(f4 acc[R / 16][2], float* act, const float bias[2], float* __restrict__ Z,
+                                          float* __restrict__ H, long long r0, int n, int c0, int l) {
+  constexpr int RT = R / 16;
+  __syncthreads();  // every wave has read the tile
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int c = c0 + 16 * t + (l & 15);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = 16 * rt + 4 * (l >> 4) + q;
+        const float z = acc[rt][t][q] + bias[t], h = gelu(z);
+        act[row * kLd + c] = h;
+        if (KEEP && r0 + row < n) {
+          Z[(r0 + row) * kHid + c] = z;
+          H[(r0 + row) * kHid + c] = h;
+        }
+      }
+  }
+  __syncthreads();
+  clear<RT>(acc);
+}
+
+template <int R, bool KEEP>
+__global__ void __launch_bounds__(kThreads) kFewWaves forward_kernel(const float* __restrict__ prm, int n,
+                                                                     const float* __restrict__ x,
+                                                                     float* __restrict__ y, float* __restrict__ work) {
+  constexpr int RT = R / 16;
+  __shared__ __align__(16) float act[R * kLd];
+  __shared__ __align__(16) float w4[kOut * kHid];
+  const long long r0 = (long long)blockIdx.x * R, L = (long long)n * kHid;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6, c0 = 32 * w;
+  const float *W1 = prm + kOffW1, *W2 = prm + kOffW2, *W3 = prm + kOffW3;
+  stage_rows<R, kIn>(act, kLdIn, x, r0, n);
+  if (threadIdx.x < kOut * kHid / 4) *reinterpret_cast<f4*>(w4 + 4 * threadIdx.x) = ld4(prm + kOffW4 + 4 * threadIdx.x);
+  const int c = c0 + (l & 15);
+  const float b1[2] = {prm[kOffB1 + c], prm[kOffB1 + c + 16]}, b2[2] = {prm[kOffB2 + c], prm[kOffB2 + c + 16]},
+              b3[2] = {prm[kOffB3 + c], prm[kOffB3 + c + 16]};
+  const int k0 = stage_k(0, w), k1 = stage_k(1, w), k2 = stage_k(2, w), k3 = stage_k(3, w);
+  Stage A, B, C;
+  wt_load<kIn, kIn / 16>(A, W1, 0, c0, l);
+  wt_load<kHid>(B, W2, k0, c0, l);
+  wt_load<kHid>(C, W2, k1, c0, l);
+  f4 acc[RT][2];
+  clear<RT>(acc);
+  __syncthreads();
+  wt_mul<RT, kIn / 16>(acc, A, act, kLdIn, 0, l);
+  wt_load<kHid>(A, W2, k2, c0, l);
+  layer_out<R, KEEP>(acc, act, b1, work, work + L, r0, n, c0, l);
+  wt_mul<RT>(acc, B, act, kLd, k0, l);
+  wt_load<kHid>(B, W2, k3, c0, l);
+  wt_mul<RT>(acc, C, act, kLd, k1, l);
+  wt_load<kHid>(C, W3, k0, c0, l);
+  wt_mul<RT>(acc, A, act, kLd, k2, l);
+  wt_load<kHid>(A, W3, k1, c0, l);
+  wt_mul<RT>(acc, B, act, kLd, k3, l);
+  wt_load<kHid>(B, W3, k2, c0, l);
+  layer_out<R, KEEP>(acc, act, b2, work + 2 * L, work + 3 * L, r0, n, c0, l);
+  wt_mul<RT>(acc, C, act, kLd, k0, l);
+  wt_load<kHid>(C, W3, k3, c0, l);
+  wt_mul<RT>(acc, A, act, kLd, k1, l);
+  wt_mul<RT>(acc, B, act, kLd, k2, l);
+  wt_mul<RT>(acc, C, act, kLd, k3, l);
+  layer_out<R, KEEP>(acc, act, b3, work + 4 * L, work + 5 * L, r0, n, c0, l);
+  // the three outputs of a row: kPer lanes, 4 values of H at a time
+  constexpr int kPer = kThreads / R;
+  const int row = threadIdx.x / kPer, part = threadIdx.x % kPer;
+  float s[kOut] = {0.f, 0.f, 0.f};
+  for (int k = 4 * part; k < kHid; k += 4 * kPer) {
+    const f4 h = *reinterpret_cast<const f4*>(act + row * kLd + k);
+#pragma unroll
+    for (int o = 0; o < kOut; ++o) {
+      const f4 v = *reinterpret_cast<const f4*>(w4 + o * kHid + k);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s[o] = fmaf(h[q], v[q], s[o]);
+    }
+  }
+#pragma unroll
+  for (int m = kPer / 2; m > 0; m >>= 1)
+#pragma unroll
+    for (int o = 0; o < kOut; ++o) s[o] += __shfl_xor(s[o], m, kPer);
+  if (part == 0 && r0 + row < n) {
+#pragma unroll
+    for (int o = 0; o < kOut; ++o) y[(r0 + row) * kOut + o] = s[o] + prm[kOffB4 + o];
+  }
+}
+
+// -------------------------------------------------------------- backward ----
+// dZ3 = (dy W4) * gelu'(Z3) into dz3, dZ2 = (dZ3 W3) * gelu'(Z2) into dz2,
+// R rows a workgroup.
+template <int R>
+__global__ void __launch_bounds__(kThreads) kFewWaves backward_rows_kernel(const float* __restrict__ prm, int n,
+                                                                 const float* __restrict__ work,
+                                                                 const float* __restrict__ dy, float* __restrict__ dz3,
+                                                                 float* __restrict__ dz2) {
+  constexpr int RT = R / 16;
+  __shared__ __align__(16) float act[R * kLd];
+  const long long r0 = (long long)blockIdx.x * R, L = (long long)n * kHid;
+  const float *Z2 = work + 2 * L, *Z3 = work + 4 * L, *W3 = prm + kOffW3;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6, c0 = 32 * w;
+  const int k0 = stage_k(0, w), k1 = stage_k(1, w), k2 = stage_k(2, w), k3 = stage_k(3, w);
+  Stage A, B, C;
+  w_load(A, W3, k0, c0, l);
+  w_load(B, W3, k1, c0, l);
+  {
+    const int c = threadIdx.x % kHid;
+    const float* W4 = prm + kOffW4;
+    const float u[kOut] = {W4[c], W4[kHid + c], W4[2 * kHid + c]};
+    for (int row = threadIdx.x / kHid; row < R; row += kThreads / kHid) {
+      float d = 0.f;
+      if (r0 + row < n) {
+        const float* dr = dy + (r0 + row) * kOut;
+#pragma unroll
+        for (int o = 0; o < kOut; ++o) d = fmaf(dr[o], u[o], d);
+        d *= gelu_grad(Z3[(r0 + row) * kHid + c]);
+        dz3[(r0 + row) * kHid + c] = d;
+      }
+      act[row * kLd + c] = d;
+    }
+  }
+  w_load(C, W3, k2, c0, l);
+  const int c = c0 + 2 * (l & 15), g = l >> 4;
+  f2 z[RT][4];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      int idx = threadIdx.x + q * kGemmThreads;
-      int rr, kk;
-      if (TA) { kk = idx / kTile; rr = idx % kTile; }
-      else { rr = idx / kTk; kk = idx % kTk; }
-      int gr = r0 + rr, gk = k0 + kk;
-      float v = 0.f;
-      if (gr < R && gk < k_end) v = TA ? A[(long long)gk * lda + gr] : A[(long long)gr * lda + gk];
-      As[kk][rr] = v;
-      int cc, kb;
-      if (TB) { cc = idx / kTk; kb = idx % kTk; }
-      else { kb = idx / kTile; cc = idx % kTile; }
-      int gc = c0 + cc, gkb = k0 + kb;
-      float w = 0.f;
-      if (gc < Cn && gkb < k_end) w = TB ? B[(long long)gc * ldb + gkb] : B[(long long)gkb * ldb + gc];
-      Bs[kb][cc] = w;
+      const long long row = r0 + 16 * rt + 4 * g + q;
+      z[rt][q] = row < n ? ld2(Z2 + row * kHid + c) : f2{0.f, 0.f};
+    }
+  __syncthreads();
+  f4 acc[RT][2];
+  clear<RT>(acc);
+  w_mul<RT>(acc, A, act, k0, l);
+  w_load(A, W3, k3, c0, l);
+  w_mul<RT>(acc, B, act, k1, l);
+  w_mul<RT>(acc, C, act, k2, l);
+  w_mul<RT>(acc, A, act, k3, l);
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long long row = r0 + 16 * rt + 4 * g + q;
+      if (row < n)
+        st2(dz2 + row * kHid + c,
+            f2{acc[rt][0][q] * gelu_grad(z[rt][q][0]), acc[rt][1][q] * gelu_grad(z[rt][q][1])});
+    }
+}
+
+// The parameter gradients, added into grad, in one launch of three kinds of
+// workgroups: 40 us for 4096 rows, where the eight launches of a VALU product
+// with three row splits (48 workgroups for 256 CUs) took 940 us. Each splits the batch rows, so that the small outputs (147k
+// values) still fill the chip; a split adds its sums with one atomic a value,
+// so there are at most kMaxSplits of them.
+//   [0, b1)        layer 1: dZ1 = (dZ2 W2) * gelu'(Z1) of 64 rows in LDS,
+//                  then dW1 += dZ1^T x and db1
+//   [b1, b1 + b23) layers 3 and 2: a 64 x 128 tile of dW += dZ^T H, its rows
+//                  split over the splits and again over four wave pairs,
+//                  summed in LDS; db from the first column tile's operand
+//   the rest       layer 4: dW4 += dy^T H3, db4
+constexpr int kRows1 = 64;
+constexpr int kTileR = 64, kTileC = 128;
+constexpr int kTiles = (kHid / kTileR) * (kHid / kTileC);  // of one layer's dW
+constexpr int kMaxSplits = 16;
+
+__device__ __forceinline__ void layer1_block(float* lds, int block, const float* __restrict__ prm, int n,
+                                             const float* __restrict__ x, const float* __restrict__ Z1,
+                                             const float* __restrict__ dz2, float* grad) {
+  constexpr int RT = kRows1 / 16;
+  float* act = lds;
+  float* xs = lds + kRows1 * kLd;
+  const long long r0 = (long long)block * kRows1;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6, c0 = 32 * w;
+  const float* W2 = prm + kOffW2;
+  const int k0 = stage_k(0, w), k1 = stage_k(1, w), k2 = stage_k(2, w), k3 = stage_k(3, w);
+  Stage A, B;
+  w_load(A, W2, k0, c0, l);
+  stage_rows<kRows1, kHid>(act, kLd, dz2, r0, n);
+  stage_rows<kRows1, kIn>(xs, kLdIn, x, r0, n);
+  w_load(B, W2, k1, c0, l);
+  __syncthreads();
+  const int j = l & 15, g = l >> 4;
+  {
+    const int c = c0 + 2 * j;
+    f4 acc[RT][2];
+    clear<RT>(acc);
+    w_mul<RT>(acc, A, act, k0, l);
+    w_load(A, W2, k2, c0, l);
+    w_mul<RT>(acc, B, act, k1, l);
+    w_load(B, W2, k3, c0, l);
+    w_mul<RT>(acc, A, act, k2, l);
+    w_mul<RT>(acc, B, act, k3, l);
+    __syncthreads();  // every wave has read the tile
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = 16 * rt + 4 * g + q;
+        f2 d = f2{0.f, 0.f};
+        if (r0 + row < n) {
+          const f2 z = ld2(Z1 + (r0 + row) * kHid + c);
+          d = f2{acc[rt][0][q] * gelu_grad(z[0]), acc[rt][1][q] * gelu_grad(z[1])};
+        }
+        *reinterpret_cast<f2*>(act + row * kLd + c) = d;
+      }
+  }
+  __syncthreads();
+  // dW1 rows [c0, c0 + 32) of this wave: 2 x 3 tiles over the 64 batch rows
+  f4 acc[2][3];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k = 0; k < kRows1; k += 4) {
+    float av[2], bv[3];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) av[a] = act[(k + g) * kLd + c0 + 16 * a + j];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) bv[b] = xs[(k + g) * kLdIn + 16 * b + j];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a], bv[b], acc[a][b], 0, 0, 0);
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        unsafeAtomicAdd(grad + kOffW1 + (c0 + 16 * a + 4 * g + q) * kIn + 16 * b + j, acc[a][b][q]);
+  if (threadIdx.x < kHid) {
+    float s = 0.f;
+    for (int r = 0; r < kRows1; ++r) s += act[r * kLd + threadIdx.x];
+    unsafeAtomicAdd(grad + kOffB1 + threadIdx.x, s);
+  }
+}
+
+__device__ __forceinline__ void dw_tile_block(float* lds, int tile, int k_begin, int k_end, const float* __restrict__ dz,
+                                              const float* __restrict__ h, float* dW, float* db) {
+  constexpr int kAhead = 4;  // pairs of batch rows loaded ahead of their use
+  const int tr0 = (tile / (kHid / kTileC)) * kTileR, tc0 = (tile % (kHid / kTileC)) * kTileC;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int sub = w & 1, ks = w >> 1;
+  const int i = l & 31, half = l >> 5;
+  const int span = (k_end - k_begin + 3) / 4;
+  const int kb = k_begin + ks * span, ke = min(k_end, kb + span);
+  const float* ap = dz + tr0 + 2 * i;
+  const float* bp = h + tc0 + 64 * sub + 2 * i;
+  f16 acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[a][b][q] = 0.f;
+  f2 sum = f2{0.f, 0.f};
+  f2 av[kAhead], bv[kAhead];
+  auto load = [&](int k, f2* a, f2* b) {
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      const int r = k + 2 * s + half;
+      a[s] = b[s] = f2{0.f, 0.f};
+      if (r < ke) {
+        a[s] = ld2(ap + (long long)r * kHid);
+        b[s] = ld2(bp + (long long)r * kHid);
+      }
+    }
+  };
+  load(kb, av, bv);
+  for (int k = kb; k < ke; k += 2 * kAhead) {
+    f2 an[kAhead], bn[kAhead];
+    load(k + 2 * kAhead, an, bn);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      sum += av[s];
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s][a], bv[s][b], acc[a][b], 0, 0, 0);
+    }
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      av[s] = an[s];
+      bv[s] = bn[s];
+    }
+  }
+  // rows tr0 + 2 m + a, columns tc0 + 64 sub + 2 i + b: the four waves of a
+  // column half are summed through LDS, one row parity at a time
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    float* mine = lds + w * (32 * 64);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int m = 8 * (q / 4) + 4 * half + q % 4;
+      *reinterpret_cast<f2*>(mine + m * 64 + 2 * i) = f2{acc[a][0][q], acc[a][1][q]};
     }
     __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < kTk; ++kk) {
-      float av[4], bv[4];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) av[a] = As[kk][tr * 4 + a];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) bv[b] = Bs[kk][tc * 4 + b];
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = fmaf(av[a], bv[b], acc[a][b]);
+    for (int e = threadIdx.x; e < 32 * kTileC; e += kThreads) {
+      const int m = e / kTileC, c = e % kTileC;
+      const float* p = lds + (c / 64) * (32 * 64) + m * 64 + c % 64;
+      const float v = (p[0] + p[2 * 32 * 64]) + (p[4 * 32 * 64] + p[6 * 32 * 64]);
+      unsafeAtomicAdd(dW + (tr0 + 2 * m + a) * kHid + tc0 + c, v);
     }
     __syncthreads();
   }
+  if (tc0 == 0) {
+    if (sub == 0) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    int r = r0 + tr * 4 + a;
-    if (r >= R) continue;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      int c = c0 + tc * 4 + b;
-      if (c >= Cn) continue;
-      long long o = (long long)r * ldc + c;
-      float v = acc[a][b];
-      if (EPI == EPI_BIAS) {
-        C[o] = v + bias[c];
-      } else if (EPI == EPI_BIAS_GELU) {
-        float z = v + bias[c];
-        P[o] = z;
-        C[o] = gelu(z);
-      } else if (EPI == EPI_GELU_BACK) {
-        C[o] = v * gelu_grad(P[o]);
-      } else {
-        unsafeAtomicAdd(C + o, v);
+      for (int b = 0; b < 2; ++b) {
+        const float s = sum[b] + __shfl_xor(sum[b], 32, 64);
+        if (half == 0) lds[ks * kTileR + 2 * i + b] = s;
       }
+    }
+    __syncthreads();
+    if (threadIdx.x < kTileR) {
+      const float* p = lds + threadIdx.x;
+      unsafeAtomicAdd(db + tr0 + threadIdx.x, (p[0] + p[kTileR]) + (p[2 * kTileR] + p[3 * kTileR]));
     }
   }
 }
 
-// Column sums of D [n][m] added into out[m] (bias gradients).
-__global__ void __launch_bounds__(256) colsum_kernel(int n, int m, const float* __restrict__ D, float* out) {
-  int c = blockIdx.x * 64 + (threadIdx.x & 63);
-  int part = threadIdx.x >> 6;  // 4 row partitions per block
-  if (c >= m) return;
-  float s = 0.f;
-  for (int r = blockIdx.y * 4 + part; r < n; r += gridDim.y * 4) s += D[(long long)r * m + c];
-  unsafeAtomicAdd(out + c, s);
+__device__ __forceinline__ void layer4_block(float* lds, int k_begin, int k_end, const float* __restrict__ dy,
+                                             const float* __restrict__ H3, float* grad) {
+  const int c = threadIdx.x % kHid, part = threadIdx.x / kHid;
+  float s[kOut] = {0.f, 0.f, 0.f}, b[kOut] = {0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int r = k_begin + part; r < k_end; r += kThreads / kHid) {
+    const float hv = H3[(long long)r * kHid + c];
+#pragma unroll
+    for (int o = 0; o < kOut; ++o) {
+      const float d = dy[(long long)r * kOut + o];
+      s[o] = fmaf(d, hv, s[o]);
+      b[o] += d;
+    }
+  }
+  if (part == 1) {
+#pragma unroll
+    for (int o = 0; o < kOut; ++o) lds[o * kHid + c] = s[o];
+    if (c == 0) {
+#pragma unroll
+      for (int o = 0; o < kOut; ++o) lds[kOut * kHid + o] = b[o];
+    }
+  }
+  __syncthreads();
+  if (part == 0) {
+#pragma unroll
+    for (int o = 0; o < kOut; ++o) unsafeAtomicAdd(grad + kOffW4 + o * kHid + c, s[o] + lds[o * kHid + c]);
+    if (c == 0) {
+#pragma unroll
+      for (int o = 0; o < kOut; ++o) unsafeAtomicAdd(grad + kOffB4 + o, b[o] + lds[kOut * kHid + o]);
+    }
+  }
+}
+
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) gradients_kernel(const float* __restrict__ prm, int n,
+                                                             const float* __restrict__ x,
+                                                             const float* __restrict__ work,
+                                                             const float* __restrict__ dy,
+                                                             const float* __restrict__ dz3,
+                                                             const float* __restrict__ dz2, float* grad, int b1,
+                                                             int b23, int chunk) {
+  __shared__ __align__(16) float lds[kRows1 * (kLd + kLdIn)];
+  static_assert(kRows1 * (kLd + kLdIn) >= 8 * 32 * 64, "the tiles' sums fit");
+  const long long L = (long long)n * kHid;
+  int blk = blockIdx.x;
+  if (blk < b1) {
+    layer1_block(lds, blk, prm, n, x, work, dz2, grad);
+    return;
+  }
+  blk -= b1;
+  if (blk < b23) {
+    // a split's tiles are neighbours, so that they share its rows in L2
+    const int split = blk / (2 * kTiles), tile = blk % (2 * kTiles);
+    const int k0 = split * chunk, k1 = min(n, k0 + chunk);
+    if (tile < kTiles) dw_tile_block(lds, tile, k0, k1, dz3, work + 3 * L, grad + kOffW3, grad + kOffB3);
+    else dw_tile_block(lds, tile - kTiles, k0, k1, dz2, work + L, grad + kOffW2, grad + kOffB2);
+    return;
+  }
+  blk -= b23;
+  layer4_block(lds, blk * chunk, min(n, (blk + 1) * chunk), dy, work + 5 * L, grad);
 }
 
 // Weighted mean squared error over [n][3]: loss += sum w_i |y_i - t_i|^2 / W,
@@ -184,72 +621,44 @@ __global__ void __launch_bounds__(256) zero_f32_kernel(long long n, float* p) {
 // --------------------------------------------------------------- launchers ----
 static inline unsigned gblocks(long long n, int bs) { return unsigned((n + bs - 1) / bs); }
 
-template <bool TA, bool TB, int EPI>
-static hipError_t gemm(int R, int Cn, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
-                       const float* bias, float* P, hipStream_t s, int splits = 1) {
-  if (R <= 0 || Cn <= 0) return hipSuccess;
-  int chunk = (K + splits - 1) / splits;
-  chunk = (chunk + kTk - 1) / kTk * kTk;
-  int zs = (K + chunk - 1) / chunk;
-  dim3 grid(gblocks(Cn, kTile), gblocks(R, kTile), zs < 1 ? 1 : zs);
-  hipLaunchKernelGGL((gemm_kernel<TA, TB, EPI>), grid, dim3(kGemmThreads), 0, s, R, Cn, K, A, lda, B, ldb, C, ldc,
-                     bias, P, chunk);
-  return hipGetLastError();
-}
+// 32 rows a workgroup halve the reads of the weights; below 256 of those
+// workgroups half of the chip would stand idle, and 16 rows are the better
+// split.
+constexpr int kWideRows = 32 * 256;
 
-#define IPC_TRY(expr)                \
-  do {                               \
-    hipError_t _e = (expr);          \
-    if (_e != hipSuccess) return _e; \
-  } while (0)
-
-hipError_t mlp_forward(const float* prm, int n, const float* x, float* y, float* work, float* tmp, hipStream_t s) {
-  // Without a work buffer (inference) the activations ping-pong in tmp.
-  long long L = (long long)n * kHid;
-  float *Z1, *H1, *Z2, *H2, *Z3, *H3;
-  if (work) {
-    Z1 = work; H1 = work + L; Z2 = work + 2 * L; H2 = work + 3 * L; Z3 = work + 4 * L; H3 = work + 5 * L;
+hipError_t mlp_forward(const float* prm, int n, const float* x, float* y, float* work, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  const dim3 block(kThreads);
+  if (n >= kWideRows) {
+    if (work) hipLaunchKernelGGL((forward_kernel<32, true>), dim3(gblocks(n, 32)), block, 0, s, prm, n, x, y, work);
+    else hipLaunchKernelGGL((forward_kernel<32, false>), dim3(gblocks(n, 32)), block, 0, s, prm, n, x, y, work);
   } else {
-    Z1 = Z2 = Z3 = tmp;
-    H1 = H3 = tmp + L;
-    H2 = tmp + 2 * L;
+    if (work) hipLaunchKernelGGL((forward_kernel<16, true>), dim3(gblocks(n, 16)), block, 0, s, prm, n, x, y, work);
+    else hipLaunchKernelGGL((forward_kernel<16, false>), dim3(gblocks(n, 16)), block, 0, s, prm, n, x, y, work);
   }
-  IPC_TRY((gemm<false, true, EPI_BIAS_GELU>(n, kHid, kIn, x, kIn, prm + kOffW1, kIn, H1, kHid, prm + kOffB1, Z1, s)));
-  IPC_TRY((gemm<false, true, EPI_BIAS_GELU>(n, kHid, kHid, H1, kHid, prm + kOffW2, kHid, H2, kHid, prm + kOffB2, Z2, s)));
-  IPC_TRY((gemm<false, true, EPI_BIAS_GELU>(n, kHid, kHid, H2, kHid, prm + kOffW3, kHid, H3, kHid, prm + kOffB3, Z3, s)));
-  return gemm<false, true, EPI_BIAS>(n, kOut, kHid, H3, kHid, prm + kOffW4, kHid, y, kOut, prm + kOffB4, nullptr, s);
+  return hipGetLastError();
 }
 
 hipError_t mlp_backward(const float* prm, int n, const float* x, const float* work, const float* dy, float* grad,
                         float* tmp, hipStream_t s) {
-  long long L = (long long)n * kHid;
-  const float *Z1 = work, *H1 = work + L, *Z2 = work + 2 * L, *H2 = work + 3 * L, *Z3 = work + 4 * L,
-              *H3 = work + 5 * L;
-  float *dA = tmp, *dB = tmp + L;
-  int splits = n / 2048 + 1;
-  if (splits > 64) splits = 64;
-  // layer 4: dW4 += dy^T H3, db4 += sum dy, dZ3 = (dy W4) * gelu'(Z3)
-  IPC_TRY((gemm<true, false, EPI_ATOMIC>(kOut, kHid, n, dy, kOut, H3, kHid, grad + kOffW4, kHid, nullptr, nullptr, s,
-                                         splits)));
-  hipLaunchKernelGGL(colsum_kernel, dim3(gblocks(kOut, 64), 32), dim3(256), 0, s, n, kOut, dy, grad + kOffB4);
-  IPC_TRY((gemm<false, false, EPI_GELU_BACK>(n, kHid, kOut, dy, kOut, prm + kOffW4, kHid, dA, kHid, nullptr,
-                                             const_cast<float*>(Z3), s)));
-  // layer 3
-  IPC_TRY((gemm<true, false, EPI_ATOMIC>(kHid, kHid, n, dA, kHid, H2, kHid, grad + kOffW3, kHid, nullptr, nullptr, s,
-                                         splits)));
-  hipLaunchKernelGGL(colsum_kernel, dim3(gblocks(kHid, 64), 32), dim3(256), 0, s, n, kHid, dA, grad + kOffB3);
-  IPC_TRY((gemm<false, false, EPI_GELU_BACK>(n, kHid, kHid, dA, kHid, prm + kOffW3, kHid, dB, kHid, nullptr,
-                                             const_cast<float*>(Z2), s)));
-  // layer 2
-  IPC_TRY((gemm<true, false, EPI_ATOMIC>(kHid, kHid, n, dB, kHid, H1, kHid, grad + kOffW2, kHid, nullptr, nullptr, s,
-                                         splits)));
-  hipLaunchKernelGGL(colsum_kernel, dim3(gblocks(kHid, 64), 32), dim3(256), 0, s, n, kHid, dB, grad + kOffB2);
-  IPC_TRY((gemm<false, false, EPI_GELU_BACK>(n, kHid, kHid, dB, kHid, prm + kOffW2, kHid, dA, kHid, nullptr,
-                                             const_cast<float*>(Z1), s)));
-  // layer 1
-  IPC_TRY((gemm<true, false, EPI_ATOMIC>(kHid, kIn, n, dA, kHid, x, kIn, grad + kOffW1, kIn, nullptr, nullptr, s,
-                                         splits)));
-  hipLaunchKernelGGL(colsum_kernel, dim3(gblocks(kHid, 64), 32), dim3(256), 0, s, n, kHid, dA, grad + kOffB1);
+  if (n <= 0) return hipSuccess;
+  const long long L = (long long)n * kHid;
+  float *dz3 = tmp, *dz2 = tmp + L;
+  if (n >= kWideRows)
+    hipLaunchKernelGGL(backward_rows_kernel<32>, dim3(gblocks(n, 32)), dim3(kThreads), 0, s, prm, n, work, dy, dz3,
+                       dz2);
+  else
+    hipLaunchKernelGGL(backward_rows_kernel<16>, dim3(gblocks(n, 16)), dim3(kThreads), 0, s, prm, n, work, dy, dz3,
+                       dz2);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  int splits = gblocks(n, 256);
+  if (splits > kMaxSplits) splits = kMaxSplits;
+  const int chunk = gblocks(n, splits);
+  splits = gblocks(n, chunk);
+  const int b1 = gblocks(n, kRows1), b23 = 2 * kTiles * splits;
+  hipLaunchKernelGGL(gradients_kernel, dim3(b1 + b23 + splits), dim3(kThreads), 0, s, prm, n, x, work, dy, dz3, dz2,
+                     grad, b1, b23, chunk);
   return hipGetLastError();
 }
 
@@ -265,37 +674,6 @@ hipError_t mlp_adam(float* p, const float* g, float* m, float* v, long long n, f
   float c1 = 1.0f - powf(b1, float(step)), c2 = 1.0f - powf(b2, float(step));
   hipLaunchKernelGGL(adam_kernel, dim3(gblocks(n, 256)), dim3(256), 0, s, n, p, g, m, v, lr, b1, b2, eps, c1, c2);
   return hipGetLastError();
-}
-
-// Device address of `scratch` on the current device, looked up once per
-// device (with that device current) and kept; nullptr with *err set when the
-// lookup fails.
-static float* scratch_on_device(hipError_t* err) {
-  constexpr int kMaxDevices = 64;
-  static std::mutex mu;
-  static float* addr[kMaxDevices] = {};
-  int dev = 0;
-  *err = hipGetDevice(&dev);
-  if (*err != hipSuccess) return nullptr;
-  if (dev < 0 || dev >= kMaxDevices) {
-    *err = hipErrorInvalidDevice;
-    return nullptr;
-  }
-  std::lock_guard<std::mutex> lock(mu);
-  if (!addr[dev]) {
-    void* p = nullptr;
-    *err = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (*err != hipSuccess) return nullptr;
-    addr[dev] = static_cast<float*>(p);
-  }
-  return addr[dev];
-}
-
-hipError_t mlp_forward_noalloc(const float* prm, int n, const float* x, float* y, hipStream_t s) {
-  hipError_t err = hipSuccess;
-  float* tmp = scratch_on_device(&err);
-  if (!tmp) return err;
-  return mlp_forward(prm, n, x, y, nullptr, tmp, s);
 }
 
 hipError_t zero_f32(float* p, long long n, hipStream_t s) {

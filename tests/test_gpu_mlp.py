@@ -69,3 +69,37 @@ def test_training_reduces_loss(dev):
     first = net.train_epochs(xt, tt, None, epochs=1, batch=1024, lr=1e-3)
     last = net.train_epochs(xt, tt, None, epochs=30, batch=1024, lr=1e-3)
     assert last < 0.2 * first
+
+
+@pytest.mark.parametrize("n", [16, 17, 63, 65, 255, 257, 4097, 8191, 8192, 8209])
+def test_row_tiles_and_splits_match_oracle(dev, n):
+    """Rows around the tiles of 16, 32 and 64, the gradient's row splits (256
+    a split, at most 16) and the change from 16 to 32 rows a workgroup at
+    8192. A sum of n products in fp32 is off by at most n 2^-24 of the sum of
+    their magnitudes; typical sums by its square root, and the bars leave ten
+    times that."""
+    rng = np.random.default_rng(n)
+    p = mlp.init(4).astype(np.float32)
+    x = rng.standard_normal((n, mlp.IN)).astype(np.float32)
+    dy = rng.standard_normal((n, mlp.OUT)).astype(np.float32)
+    net = warmstart.MLP(dev, params=torch.from_numpy(p).to(dev))
+    xt = torch.from_numpy(x).to(dev)
+    y, work = net.forward(xt, keep=True)
+    y2, _ = net.forward(xt)
+    grad = torch.zeros_like(net.params)
+    net.backward(xt, work, torch.from_numpy(dy).to(dev), grad)
+    torch.cuda.synchronize()
+    yr, cache = mlp.forward(p.astype(np.float64), x.astype(np.float64))
+    gr = mlp.backward(p.astype(np.float64), cache, dy.astype(np.float64))
+    assert torch.equal(y, y2)
+    assert np.abs(y.cpu().numpy() - yr).max() <= 10 * 2.0 ** -24 * 16 * np.abs(yr).max()
+    kept = work.cpu().numpy().reshape(6, n, mlp.HID)
+    for k in range(6):
+        assert np.abs(kept[k] - cache[1 + k]).max() <= 10 * 2.0 ** -24 * 16 * np.abs(cache[1 + k]).max()
+    gg = grad.cpu().numpy().astype(np.float64)
+    o = 0
+    for name, shape in mlp.SHAPES:
+        k = int(np.prod(shape))
+        a, b = gg[o:o + k], gr[o:o + k]
+        assert np.linalg.norm(a - b) <= 10 * 2.0 ** -24 * np.sqrt(max(n, 256)) * np.linalg.norm(b), name
+        o += k
