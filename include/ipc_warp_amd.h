@@ -442,8 +442,7 @@ int ipc_bsr_mv(int n_rows, const int* offsets, const int* columns, const float* 
  * x (float [n_rows][3]), stopping when |r| <= tol |b| (checked on the host
  * every check_every iterations, default 10, as the reference's cg does) or
  * after maxiter iterations (<= 0: 3 n_rows); iterations run in whole groups
- * of check_every rounded up to even, captured once as a HIP graph for the
- * given pointers and size and replayed. jacobi != 0 preconditions with
+ * of check_every rounded up to even. jacobi != 0 preconditions with
  * the inverse diagonal of the diagonal blocks. Vectors are fp32, dot
  * products fp64 and summed in a fixed order. Writes the iteration count of
  * the last check and |r| there. Synchronises `stream` at each check. An

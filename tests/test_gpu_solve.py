@@ -104,3 +104,37 @@ def test_cg_graph_replays_are_identical(dev, system):
     for it, res, x in outs[1:]:
         assert it == outs[0][0] and res == outs[0][1]
         assert np.array_equal(x.view(np.uint32), outs[0][2].view(np.uint32))
+
+
+@pytest.mark.parametrize("jacobi", [False, True])
+@pytest.mark.parametrize("rows,width", [(1, 0), (2, 1), (63, 3), (64, 15), (65, 16), (513, 17), (2049, 40),
+                                        (262144 + 77, 2)])
+def test_cg_row_lengths_and_grid_strides(dev, rows, width, jacobi):
+    """Diagonally dominant banded systems: rows of 1 to 2 width + 1 blocks
+    (a lane takes two of every 16 at a time), row counts around a workgroup's
+    64 rows and past the 4096 workgroups of the product. The matrix's
+    spectrum lies within [1, 3] times its diagonal's range of [1, 2], so that
+    |x - x*| <= |r| / 1 <= tol |b|; fp32 adds what the residual recurrence
+    rounds, a few 1e-7 of |x| an iteration."""
+    rng = np.random.default_rng(rows + width)
+    reach = rng.integers(0, width + 1, rows)
+    i = np.repeat(np.arange(rows), reach)
+    j = i + 1 + np.concatenate([np.arange(k) for k in reach]) if i.size else i
+    i, j = i[j < rows], j[j < rows]
+    B = rng.uniform(-1, 1, (i.size, 3, 3)) / (3 * max(2 * width, 1))
+    d = rng.uniform(2, 4, (rows, 3, 1)) * np.eye(3)
+    r = np.concatenate([np.arange(rows), i, j]).astype(np.int32)
+    c = np.concatenate([np.arange(rows), j, i]).astype(np.int32)
+    v = np.concatenate([d, B, B.transpose(0, 2, 1)]).astype(np.float32)
+    A = sparse.bsr_from_triplets(rows, rows, *(torch.from_numpy(a).to(dev) for a in (r, c, v)))
+    full = (3 * np.repeat(r, 9).astype(np.int64) + np.tile(np.repeat(np.arange(3), 3), r.size),
+            3 * np.repeat(c, 9).astype(np.int64) + np.tile(np.tile(np.arange(3), 3), c.size))
+    ref = sp.coo_matrix((v.reshape(-1).astype(np.float64), full), shape=(3 * rows, 3 * rows)).tocsr()
+    want = rng.normal(size=3 * rows)
+    b = torch.from_numpy((ref @ want).reshape(rows, 3).astype(np.float32)).to(dev)
+    x = torch.zeros_like(b)
+    it, res, goal = sparse.cg(A, b, x, tol=1e-6, maxiter=200, jacobi=jacobi)
+    torch.cuda.synchronize()
+    assert 0 < it < 200 and it % 2 == 0 and res <= goal
+    err = np.linalg.norm(x.cpu().numpy().reshape(-1) - want)
+    assert err <= 2e-6 * np.linalg.norm(b.cpu().numpy()) + 3e-7 * it * np.linalg.norm(want)
