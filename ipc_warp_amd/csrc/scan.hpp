@@ -1,6 +1,6 @@
 // Device-wide int helpers shared by the assembly and active-set code: a fill
-// kernel and an exclusive prefix sum in tiles of 4096 (256 lanes x 16),
-// then the tile sums, then the tile offsets added. Internal linkage: every
+// kernel and an exclusive prefix sum in tiles of 4096 (256 lanes x 16), then
+// the tile offsets added. Internal linkage: every
 // translation unit that includes this keeps its own copy of the kernels.
 #pragma once
 
@@ -27,75 +27,79 @@ hipError_t fill_i32(int* p, int n, int v, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Exclusive prefix of v over the workgroup's 256 lanes; sh holds 4 ints.
 __device__ int block_exclusive(int v, int* sh, int& total) {
-  const int tid = threadIdx.x;
-  sh[tid] = v;
-  __syncthreads();
-  for (int d = 1; d < kScanB; d <<= 1) {
-    const int u = tid >= d ? sh[tid - d] : 0;
-    __syncthreads();
-    sh[tid] += u;
-    __syncthreads();
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int x = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(x, d, 64);
+    x += lane >= d ? u : 0;
   }
-  total = sh[kScanB - 1];
-  const int r = sh[tid] - v;
+  __syncthreads();  // sh may still be read from the call before
+  if (lane == 63) sh[w] = x;
   __syncthreads();
-  return r;
+  const int s0 = sh[0], s1 = sh[1], s2 = sh[2], s3 = sh[3];
+  total = s0 + s1 + s2 + s3;
+  return x - v + (w > 0 ? s0 : 0) + (w > 1 ? s1 : 0) + (w > 2 ? s2 : 0);
 }
 
 __global__ __launch_bounds__(kScanB) void scan_tiles_kernel(const int* in, int n, int* out, int* tile_sum) {
-  __shared__ int sh[kScanB];
+  __shared__ int sh[4];
   const long long base = (long long)blockIdx.x * kScanTile + threadIdx.x * kScanPer;
   int v[kScanPer];
   int acc = 0;
+  if (base + kScanPer <= n) {
+    __builtin_memcpy(v, in + base, sizeof(v));
+  } else {
 #pragma unroll
-  for (int k = 0; k < kScanPer; ++k) {
-    v[k] = base + k < n ? in[base + k] : 0;
-    acc += v[k];
+    for (int k = 0; k < kScanPer; ++k) v[k] = base + k < n ? in[base + k] : 0;
   }
+#pragma unroll
+  for (int k = 0; k < kScanPer; ++k) acc += v[k];
   int total;
   int run = block_exclusive(acc, sh, total);
 #pragma unroll
   for (int k = 0; k < kScanPer; ++k) {
-    if (base + k < n) out[base + k] = run;
-    run += v[k];
+    const int x = v[k];
+    v[k] = run;
+    run += x;
+  }
+  if (base + kScanPer <= n) {
+    __builtin_memcpy(out + base, v, sizeof(v));
+  } else {
+#pragma unroll
+    for (int k = 0; k < kScanPer; ++k)
+      if (base + k < n) out[base + k] = v[k];
   }
   if (threadIdx.x == 0) tile_sum[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(kScanB) void scan_sums_kernel(int* tile_sum, int nt) {
-  __shared__ int sh[kScanB];
-  int carry = 0;
-  for (int b = 0; b < nt; b += kScanB) {
-    const int i = b + threadIdx.x;
-    const int v = i < nt ? tile_sum[i] : 0;
-    int total;
-    const int e = block_exclusive(v, sh, total);
-    if (i < nt) tile_sum[i] = carry + e;
-    carry += total;
-  }
-}
-
+// Adds to each tile past the first what the tiles before it sum to; every
+// workgroup adds those sums itself (there are few), which saves the launch
+// of a scan of theirs.
 __global__ void scan_add_kernel(int* out, int n, const int* tile_sum) {
+  __shared__ int sh[4];
   const int tile = blockIdx.x + 1;
-  const int add = tile_sum[tile];
-  const long long base = (long long)tile * kScanTile;
-  for (int k = threadIdx.x; k < kScanTile; k += kScanB)
-    if (base + k < n) out[base + k] += add;
+  int part = 0;
+  for (int i = threadIdx.x; i < tile; i += kScanB) part += tile_sum[i];
+  int add;
+  block_exclusive(part, sh, add);
+  const long long base = (long long)tile * kScanTile + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kScanPer; ++k)
+    if (base + k * kScanB < n) out[base + k * kScanB] += add;
 }
 
 // out[0..n) = exclusive prefix sums of in[0..n); in and out distinct. `part`
 // holds one int per tile.
 hipError_t exclusive_scan(const int* in, int n, int* out, DevBuf& part, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  const int nt = (n + kScanTile - 1) / kScanTile;
+  const int nt = int(((long long)n + kScanTile - 1) / kScanTile);
   hipError_t e = part.ensure(sizeof(int) * size_t(nt));
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(scan_tiles_kernel, dim3(nt), dim3(kScanB), 0, s, in, n, out, part.as<int>());
-  if (nt > 1) {
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kScanB), 0, s, part.as<int>(), nt);
-    hipLaunchKernelGGL(scan_add_kernel, dim3(nt - 1), dim3(kScanB), 0, s, out, n, part.as<int>());
-  }
+  if (nt > 1) hipLaunchKernelGGL(scan_add_kernel, dim3(nt - 1), dim3(kScanB), 0, s, out, n, part.as<int>());
   return hipGetLastError();
 }
 

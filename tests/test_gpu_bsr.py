@@ -231,3 +231,39 @@ def test_few_long_rows(dev, oracle):
     torch.cuda.synchronize()
     _say(f"bsr few long rows: {time.perf_counter() - t0:.4f} s")
     _same(_host(M), oracle.bsr_from_triplets(8, 32, rows, cols, vals))
+
+
+@pytest.mark.parametrize("columns", [1, 9, 700, 40000])
+def test_row_length_edges(dev, oracle, columns):
+    """Rows around what one wave sorts in one, two and four registers a lane
+    (64, 128, 256), around a workgroup's merges in LDS (512, 8192) and past
+    them, with few and many distinct columns, their triplets dealt at random
+    over the list; exact against the oracle (same order of the sums)."""
+    rng = np.random.default_rng(columns)
+    lengths = [0, 1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1023, 4097, 8191, 8192, 8193, 16384,
+               16385, 40001]
+    rows = np.repeat(np.arange(len(lengths)), lengths).astype(np.int32)
+    rng.shuffle(rows)
+    cols = rng.integers(0, columns, rows.size).astype(np.int32)
+    vals = rng.normal(size=(rows.size, 3, 3)).astype(np.float32)
+    M = sparse.bsr_from_triplets(len(lengths), columns, *_to_dev(dev, rows, cols, vals))
+    ref = oracle.bsr_from_triplets(len(lengths), columns, rows, cols, vals)
+    _same(_host(M), ref)
+    M.refill(torch.from_numpy(2 * vals).to(dev))
+    _same(_host(M), (ref[0], ref[1], 2 * np.asarray(ref[2])))
+
+
+@pytest.mark.parametrize("n_rows", [1, 4095, 4096, 4097, 300001])
+def test_row_count_edges(dev, oracle, n_rows):
+    """Row counts around a tile of the prefix sums (4096) and many tiles;
+    triplet counts that leave a partial tile of the count (1024), runs of
+    equal rows across its waves, and every row of a tile distinct."""
+    rng = np.random.default_rng(n_rows)
+    n = 3 * 1024 + 77
+    rows = np.concatenate([np.repeat(rng.integers(0, n_rows, 300), 7), rng.permutation(n_rows)[:1500],
+                           rng.integers(-1, n_rows + 1, n)]).astype(np.int32)
+    cols = rng.integers(0, 50, rows.size).astype(np.int32)
+    vals = rng.normal(size=(rows.size, 3, 3)).astype(np.float32)
+    vals[rng.random(rows.size) < 0.3] = 0.0
+    M = sparse.bsr_from_triplets(n_rows, 50, *_to_dev(dev, rows, cols, vals))
+    _same(_host(M), oracle.bsr_from_triplets(n_rows, 50, rows, cols, vals))
