@@ -529,18 +529,25 @@ __device__ __forceinline__ bool fixed_accept(const FixedArgs& A, const TaskPrim&
 // in bounds). The grid is persistent (tasks are counted on the device) and
 // each wave strides over groups of eight tasks, so every lane of a wave runs
 // the same trip count.
+//
+// Accepted pairs are staged per wave. A persistent workgroup finds far more
+// pairs than one stage holds (on the screw and nut 3.2 million candidates),
+// and past a full stage that is written once at the end every step with a hit
+// made a global atomicAdd of its own; those on one address serialise at about
+// 10 ns, and the CCD query took 2.09 ms, of which 0.27 are left.
+constexpr int kFixedStage = 192;  // 128 a wave: CCD query 331 us
 struct FixedSmem {
   unsigned long long stack[kGroupsPerBlock][kMaskStack];
-  BlockStage stage;
+  WaveStageN<kFixedStage> stage;
 };
 
 // Workgroup `bid` of the `nblk` serving A.
 template <int MODE>
 __device__ __forceinline__ void fixed_query_block(const FixedArgs& A, int bid, int nblk, FixedSmem& sm) {
   auto& stack = sm.stack;
-  BlockStage& stage = sm.stage;
+  auto& stage = sm.stage;
   const StageOut out{A.rec, A.ids, A.count, A.capacity};
-  stage_begin(stage);
+  int staged = 0;
   const int tid = threadIdx.x;
   const int grp = tid / kFan, r = tid % kFan;
   const int lane = __lane_id();
@@ -651,11 +658,11 @@ __device__ __forceinline__ void fixed_query_block(const FixedArgs& A, int bid, i
       bool want = false;
       int4 rec = make_int4(0, 0, 0, 0);
       if (L == 1 && hit) want = fixed_accept<MODE>(A, P, lv, rec);
-      stage_append(stage, out, want, rec, make_int2(P.src, lv.w));
+      wave_stage_append(stage, out, staged, want, rec, make_int2(P.src, lv.w));
       if (!__any(sp > 0)) break;
     }
   }
-  stage_flush(stage, out);
+  wave_stage_flush(stage, out, staged);
 }
 
 template <int MODE>
@@ -664,9 +671,11 @@ __global__ void __launch_bounds__(kQueryBlock) fixed_query_kernel(FixedArgs A) {
   fixed_query_block<MODE>(A, blockIdx.x, gridDim.x, sm);
 }
 
-// Workgroups [0, blocks_a) serve A, the rest B.
+// Workgroups [0, blocks_a) serve A, the rest B. Seven waves a SIMD are what
+// the stages leave room for in LDS; the CCD pair spills 7 registers for them
+// outside its loop (at 114 registers and four waves it took 297 us, not 274).
 template <int MA, int MB>
-__global__ void __launch_bounds__(kQueryBlock) fixed_query_pair_kernel(FixedArgs A, FixedArgs B, int blocks_a) {
+__global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_eu(7))) fixed_query_pair_kernel(FixedArgs A, FixedArgs B, int blocks_a) {
   __shared__ FixedSmem sm;
   if (int(blockIdx.x) < blocks_a) fixed_query_block<MA>(A, blockIdx.x, blocks_a, sm);
   else fixed_query_block<MB>(B, blockIdx.x - blocks_a, gridDim.x - blocks_a, sm);
@@ -698,7 +707,8 @@ FixedArgs fixed_args(const FixedQuery& q) {
 }
 
 // Persistent grid of a query: one workgroup per 32 tasks of capacity, at
-// most 2048.
+// most 2048 (1024 would fill the device once; twice that evens out the tasks'
+// lengths: the screw and nut's DCD query 237 -> 209 us).
 int fixed_blocks(const FixedQuery& q) {
   int blocks = (q.task_cap + kGroupsPerBlock - 1) / kGroupsPerBlock;
   return blocks > 2048 ? 2048 : blocks;

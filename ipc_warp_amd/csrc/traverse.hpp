@@ -116,4 +116,70 @@ __device__ __forceinline__ void stage_flush(Stage& S, const StageOut& O) {
   }
 }
 
+// The same for workgroups that go on to further queries, N pairs a wave: a
+// wave whose part is full writes it out with one global atomicAdd and goes
+// on, without waiting for the others. `n` is the wave's count, kept in a
+// register by each of its lanes.
+template <int N>
+struct WaveStageN {
+  static constexpr int kCap = N;
+  int4 rec[kQueryBlock / 64][N];
+  int2 ids[kQueryBlock / 64][N];
+  int part[kQueryBlock / 64 + 1];
+};
+
+template <typename Stage>
+__device__ __forceinline__ void wave_stage_write(const Stage& S, const StageOut& O, int n, int base) {
+  const int lane = __lane_id(), w = threadIdx.x >> 6;
+  for (int k = lane; k < n; k += 64) {
+    const int o = base + k;
+    if (o < O.capacity) {
+      if (O.rec) O.rec[o] = S.rec[w][k];
+      if (O.ids) O.ids[o] = S.ids[w][k];
+    }
+  }
+}
+
+// Called by every lane of a wave together.
+template <typename Stage>
+__device__ __forceinline__ void wave_stage_append(Stage& S, const StageOut& O, int& n, bool want, int4 rec, int2 id) {
+  const unsigned long long m = __ballot(want);
+  if (m == 0ull) return;
+  const int k = __popcll(m), lane = __lane_id(), w = threadIdx.x >> 6;
+  if (n + k > Stage::kCap) {
+    int base = 0;
+    if (lane == 0) base = atomicAdd(O.count, n);
+    base = __shfl(base, 0, 64);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    wave_stage_write(S, O, n, base);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    n = 0;
+  }
+  if (want) {
+    const int s = n + __popcll(m & ((1ull << lane) - 1ull));
+    S.rec[w][s] = rec;
+    S.ids[w][s] = id;
+  }
+  n += k;
+}
+
+// Called by the whole workgroup once every wave has finished appending: one
+// global atomicAdd for what the four parts still hold.
+template <typename Stage>
+__device__ __forceinline__ void wave_stage_flush(Stage& S, const StageOut& O, int n) {
+  constexpr int kW = kQueryBlock / 64;
+  const int w = threadIdx.x >> 6;
+  if (__lane_id() == 0) S.part[w] = n;
+  __syncthreads();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int u = 0; u < kW; ++u) {
+    before += u < w ? S.part[u] : 0;
+    total += S.part[u];
+  }
+  if (threadIdx.x == 0) S.part[kW] = total ? atomicAdd(O.count, total) : 0;
+  __syncthreads();
+  wave_stage_write(S, O, n, S.part[kW] + before);
+}
+
 }  // namespace ipcd

@@ -130,3 +130,25 @@ def test_fixed_argument_checks(dev):
         S.initialize_fixed_body_bvhs(torch.from_numpy(q[:4]).to(dev), n_bodies=1)  # body ids beyond n_bodies
     with pytest.raises(ValueError):
         S.initialize_fixed_body_bvhs(torch.from_numpy(q).to(dev).double())
+
+
+@pytest.mark.parametrize("n_theta,rows", [(48, 16), (96, 16)])
+def test_full_stages_keep_every_candidate(dev, oracle, n_theta, rows):
+    """The screw in its nut, where a wave of the persistent query fills its
+    stage of 192 pairs many times over: the contacts equal the oracle's
+    world-space sets, the bound and counts of candidates repeat from call to
+    call, and the candidates' earliest impact is the world path's."""
+    soup, q, dq, dx, fixed = scenes.screw_and_nut(seed=3, n_theta=n_theta, n_theta_nut=n_theta - 5, rows=rows)
+    S = _solver(dev, soup, q, fixed=fixed)
+    n_ee, n_pt = _check_dcd(S, soup, oracle)
+    assert n_ee > 0 and n_pt > 0
+    dxt, dqt = torch.from_numpy(dx).to(dev), torch.from_numpy(dq).to(dev)
+    seen = set()
+    for _ in range(3):
+        toi, fell_back = S.raw_toi_fixed(dxt, dqt)
+        assert not fell_back
+        seen.add((toi, *S.last_ccd_counts()))
+    assert len(seen) == 1
+    (toi, n_ee, n_pt), = seen
+    assert n_ee + n_pt > 100 * 192
+    assert toi == S.raw_toi(dxt)
