@@ -14,12 +14,13 @@
 //            each workgroup setting the distinct pairs of its triplets once;
 //   pattern  the pairs as a BSR over bodies (rows sorted) and its DOF-level
 //            BSR: body pair (A, B) owns the 16 blocks (4A + a, 4B + c);
-//   reduce   each wave walks a contiguous run of vertex triplets, each lane
-//            a fixed stride of it, summing its blocks in fp32 registers
-//            while its body pair stays the same; on a change the wave adds
-//            the lanes' sums per body pair (lane order, fp32) into one of
-//            up to 64 fp64 accumulator copies (wave index modulo the copy
-//            count) with one atomic per value;
+//   reduce   each workgroup walks a contiguous run of vertex triplets, its
+//            kept ones queued densely in order; its four waves go through
+//            the queue together, wave a summing the blocks (a, 0..3) in fp32
+//            registers while a lane's body pair stays the same; on a change
+//            the wave adds the lanes' sums per body pair (lane order, fp32)
+//            into one of up to 64 fp64 accumulator copies (workgroup index
+//            modulo the copy count) with one atomic per value;
 //   finish   values = scale * (sum of the copies) rounded to fp32.
 // The forces reduce the same way per vertex (one body per vertex).
 #include <cstdio>
@@ -27,6 +28,7 @@
 #include "../../include/ipc_warp_amd.h"
 #include "cull.hpp"
 #include "ipc_kernels.hpp"
+#include "scan.hpp"
 
 using namespace ipcd;
 
@@ -45,7 +47,6 @@ namespace {
 
 constexpr int kB = 256;
 constexpr int kWaves = kB / 64;
-constexpr int kScanTile = kB * 16;
 constexpr int kMaxBodies = 8192;
 
 int abd_fail(int code, const char* what) {
@@ -86,117 +87,72 @@ hipError_t zero_f64(double* p, long long n, hipStream_t s) {
   return hipGetLastError();
 }
 
-// exclusive scan of n ints (one tile per block, tile sums, tile offsets)
-__device__ int block_exclusive(int v, int* sh, int& total) {
-  const int tid = threadIdx.x;
-  sh[tid] = v;
-  __syncthreads();
-  for (int d = 1; d < kB; d <<= 1) {
-    const int u = tid >= d ? sh[tid - d] : 0;
-    __syncthreads();
-    sh[tid] += u;
-    __syncthreads();
-  }
-  total = sh[kB - 1];
-  const int r = sh[tid] - v;
-  __syncthreads();
-  return r;
-}
-
-__global__ __launch_bounds__(kB) void scan_tiles_kernel(const int* in, int n, int* out, int* tile_sum) {
-  __shared__ int sh[kB];
-  const long long base = (long long)blockIdx.x * kScanTile + threadIdx.x * 16;
-  int v[16];
-  int acc = 0;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    v[k] = base + k < n ? in[base + k] : 0;
-    acc += v[k];
-  }
-  int total;
-  int run = block_exclusive(acc, sh, total);
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    if (base + k < n) out[base + k] = run;
-    run += v[k];
-  }
-  if (threadIdx.x == 0) tile_sum[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(kB) void scan_sums_kernel(int* tile_sum, int nt) {
-  __shared__ int sh[kB];
-  int carry = 0;
-  for (int b = 0; b < nt; b += kB) {
-    const int i = b + threadIdx.x;
-    const int v = i < nt ? tile_sum[i] : 0;
-    int total;
-    const int e = block_exclusive(v, sh, total);
-    if (i < nt) tile_sum[i] = carry + e;
-    carry += total;
-  }
-}
-
-__global__ void scan_add_kernel(int* out, int n, const int* tile_sum) {
-  const int tile = blockIdx.x + 1;
-  const int add = tile_sum[tile];
-  const long long base = (long long)tile * kScanTile;
-  for (int k = threadIdx.x; k < kScanTile; k += kB)
-    if (base + k < n) out[base + k] += add;
-}
-
-hipError_t exclusive_scan(const int* in, int n, int* out, DevBuf& part, hipStream_t s) {
-  const int nt = nblk(n, kScanTile);
-  hipError_t e = part.ensure(sizeof(int) * size_t(nt));
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(scan_tiles_kernel, dim3(nt), dim3(kB), 0, s, in, n, out, part.as<int>());
-  if (nt > 1) {
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kB), 0, s, part.as<int>(), nt);
-    hipLaunchKernelGGL(scan_add_kernel, dim3(nt - 1), dim3(kB), 0, s, out, n, part.as<int>());
-  }
-  return hipGetLastError();
-}
-
-// The body pair of a kept vertex triplet, or -1: in range, both bodies free,
-// some value nonzero.
-__device__ inline bool triplet_pair(const int* rows, const int* cols, const float* vals, int t, int nv, int nb,
-                                    const int* body, const int* fixed, int& bi, int& bj) {
-  const int r = rows[t], c = cols[t];
+// The body pair of a vertex triplet in range with both bodies free.
+__device__ inline bool free_pair(int r, int c, int nv, int nb, const int* __restrict__ body,
+                                 const int* __restrict__ fixed, int& bi, int& bj) {
   if (unsigned(r) >= unsigned(nv) || unsigned(c) >= unsigned(nv)) return false;
   bi = body[r];
   bj = body[c];
-  if (unsigned(bi) >= unsigned(nb) || unsigned(bj) >= unsigned(nb) || fixed[bi] || fixed[bj]) return false;
+  return unsigned(bi) < unsigned(nb) && unsigned(bj) < unsigned(nb) && !fixed[bi] && !fixed[bj];
+}
+
+__device__ inline bool any_nonzero(const float* __restrict__ v) {
+  float h[9];
+  __builtin_memcpy(h, v, sizeof(h));
   bool nz = false;
 #pragma unroll
-  for (int k = 0; k < 9; ++k) nz |= !(vals[9ll * t + k] == 0.0f);
+  for (int k = 0; k < 9; ++k) nz |= !(h[k] == 0.0f);
   return nz;
 }
 
-constexpr int kMarkPer = 64;     // triplets per thread of the mark kernel
+constexpr int kMarkPer = 32;     // triplets per thread of the mark kernel
 constexpr int kMarkSet = 256;    // LDS set of body pairs per workgroup
+constexpr int kMarkProbes = 16;
 
 // Bits of the body pairs receiving a nonzero block. Each workgroup collects
 // the distinct pairs of its kB * kMarkPer triplets in an LDS set and sets
-// each bit once; a pair that finds the set full sets its bit itself.
-__global__ __launch_bounds__(kB) void mark_kernel(const int* rows, const int* cols, const float* vals, int m, int nv,
-                                                  int nb, const int* body, const int* fixed, int words,
-                                                  unsigned* bits) {
+// each bit once; a pair that finds the set full sets its bit itself. A
+// triplet whose pair is in the set already needs no look at its values: a
+// list of few body pairs is then read without them (screw and nut, 9.95
+// million triplets: 189 us with them, 50 without).
+__global__ __launch_bounds__(kB) void mark_kernel(const int* __restrict__ rows, const int* __restrict__ cols,
+                                                  const float* __restrict__ vals, int m, int nv, int nb,
+                                                  const int* __restrict__ body, const int* __restrict__ fixed,
+                                                  int words, unsigned* bits) {
   __shared__ unsigned set[kMarkSet];
   for (int i = threadIdx.x; i < kMarkSet; i += kB) set[i] = 0xffffffffu;
   __syncthreads();
-  const long long base = (long long)blockIdx.x * kB * kMarkPer;
-  for (int k = 0; k < kMarkPer; ++k) {
-    const long long t = base + (long long)k * kB + threadIdx.x;
-    int bi, bj;
-    if (t >= m || !triplet_pair(rows, cols, vals, int(t), nv, nb, body, fixed, bi, bj)) continue;
-    const unsigned key = unsigned(bi) * unsigned(nb) + unsigned(bj);
-    unsigned h = (key * 2654435761u) >> 24;  // 8 bits: kMarkSet slots
-    bool placed = false;
-    for (int probe = 0; probe < 16 && !placed; ++probe) {
-      const unsigned slot = (h + probe) & (kMarkSet - 1);
-      const unsigned old = atomicCAS(&set[slot], 0xffffffffu, key);
-      placed = old == 0xffffffffu || old == key;
+  const long long base = (long long)blockIdx.x * kB * kMarkPer + threadIdx.x;
+  constexpr int kAhead = 4;
+  for (int k0 = 0; k0 < kMarkPer; k0 += kAhead) {
+    int r[kAhead], c[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const long long t = base + (long long)(k0 + k) * kB;
+      r[k] = t < m ? rows[t] : -1;
+      c[k] = t < m ? cols[t] : -1;
     }
-    if (!placed) atomicOr(bits + (long long)bi * words + (bj >> 5), 1u << (bj & 31));
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      int bi, bj;
+      if (!free_pair(r[k], c[k], nv, nb, body, fixed, bi, bj)) continue;
+      const unsigned key = unsigned(bi) * unsigned(nb) + unsigned(bj);
+      const unsigned h = (key * 2654435761u) >> 24;  // 8 bits: kMarkSet slots
+      bool known = false;
+      for (int probe = 0; probe < kMarkProbes && !known; ++probe) {
+        const unsigned old = __hip_atomic_load(&set[(h + probe) & (kMarkSet - 1)], __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (old == 0xffffffffu) break;
+        known = old == key;
+      }
+      if (known || !any_nonzero(vals + 9 * (base + (long long)(k0 + k) * kB))) continue;
+      bool placed = false;
+      for (int probe = 0; probe < kMarkProbes && !placed; ++probe) {
+        const unsigned old = atomicCAS(&set[(h + probe) & (kMarkSet - 1)], 0xffffffffu, key);
+        placed = old == 0xffffffffu || old == key;
+      }
+      if (!placed) atomicOr(bits + (long long)bi * words + (bj >> 5), 1u << (bj & 31));
+    }
   }
   __syncthreads();
   for (int i = threadIdx.x; i < kMarkSet; i += kB) {
@@ -271,14 +227,14 @@ __device__ inline float wave_sum(float v) {
 }
 
 constexpr int kPad = 65;    // LDS row pitch of the flush table (conflict-free both ways)
-constexpr int kChunk = 48;  // values per LDS pass of a flush (3 passes of the 144)
+constexpr int kChunk = 12;  // values per LDS pass of a flush (3 passes of a wave's 36)
 
-// Adds every pending lane sum into the accumulator, one body pair at a time:
-// per pass of 48 values the lanes of that pair write their sums to LDS
-// (others write zeros), then lane k < 48 adds value k over the 64 lanes in
-// lane order and issues the fp64 atomic. `out` is this wave's accumulator
-// copy.
-__device__ void flush_pairs(int& cur_a, int cur_b, float* acc, int lane, const int* poff, const int* pcol,
+// Adds every pending lane sum of block row a into the accumulator, one body
+// pair at a time: per pass of kChunk values the lanes of that pair write
+// their sums to LDS (others write zeros), then lane k < kChunk adds value k
+// over the 64 lanes in lane order and issues the fp64 atomic. `out` is this
+// workgroup's accumulator copy.
+__device__ void flush_pairs(int& cur_a, int cur_b, float* acc, int lane, int a, const int* poff, const int* pcol,
                             float* sh, double* out) {
   while (true) {
     const unsigned long long pend = __ballot(cur_a >= 0);
@@ -286,74 +242,129 @@ __device__ void flush_pairs(int& cur_a, int cur_b, float* acc, int lane, const i
     const int leader = __ffsll(static_cast<long long>(pend)) - 1;
     const int A = __shfl(cur_a, leader), B = __shfl(cur_b, leader);
     const bool mine = cur_a == A && cur_b == B;
+    const long long first = dof_block(poff, pcol, A, B, a, 0);
 #pragma unroll
-    for (int c = 0; c < 144 / kChunk; ++c) {
+    for (int c = 0; c < 36 / kChunk; ++c) {
 #pragma unroll
       for (int k = 0; k < kChunk; ++k) sh[k * kPad + lane] = mine ? acc[c * kChunk + k] : 0.0f;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       if (lane < kChunk) {
         float sum = 0.0f;
+#pragma unroll 16
         for (int j = 0; j < 64; ++j) sum += sh[lane * kPad + j];
-        const int k = c * kChunk + lane;
-        const int blk = k / 9, e = k - 9 * blk;
-        const long long o = dof_block(poff, pcol, A, B, blk >> 2, blk & 3);
-        atomicAdd(out + 9 * o + e, static_cast<double>(sum));
+        atomicAdd(out + 9 * first + c * kChunk + lane, static_cast<double>(sum));  // the four blocks are neighbours
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     if (mine) {
       cur_a = -1;
 #pragma unroll
-      for (int k = 0; k < 144; ++k) acc[k] = 0.0f;
+      for (int k = 0; k < 36; ++k) acc[k] = 0.0f;
     }
   }
 }
 
-// One wave per block, each a contiguous run of per_wave triplets.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void reduce_hessian_kernel(const int* rows, const int* cols, const float* vals, int m,
-                                                            int per_wave, int nv, int nb, const int* body,
-                                                            const int* fixed, const float* rest, const int* poff,
-                                                            const int* pcol, double* acc_reps, int reps,
+// What bounds it: the triplets are read once, but a triplet waits for its
+// vertices, their bodies and its values in turn, and three in four of a
+// contact list with a fixed body are dropped. With one lane a triplet and all
+// 144 sums in its registers two waves a SIMD did not hide that (289 us for
+// 9.95 million triplets); here the kept ones are first queued, and a wave
+// holds 36 sums, so that five waves a SIMD run (186 us).
+constexpr int kQueuePer = 4;
+constexpr int kQueueTile = kB * kQueuePer;
+__global__ __launch_bounds__(kB) void reduce_hessian_kernel(const int* __restrict__ rows,
+                                                            const int* __restrict__ cols,
+                                                            const float* __restrict__ vals, int m, int per_block,
+                                                            int nv, int nb, const int* __restrict__ body,
+                                                            const int* __restrict__ fixed,
+                                                            const float* __restrict__ rest,
+                                                            const int* __restrict__ poff,
+                                                            const int* __restrict__ pcol, double* acc_reps, int reps,
                                                             long long rep_stride) {
-  __shared__ float sh[kChunk * kPad];
-  const int lane = threadIdx.x;
-  // waves spread their atomics over `reps` copies of the accumulator, so a
-  // body pair shared by every wave is not one chain of atomics per value
+  __shared__ int queue[2][kQueueTile];
+  __shared__ int num[2][kQueuePer * kWaves];
+  __shared__ float sh[kWaves][kChunk * kPad];
+  const int lane = threadIdx.x & 63;
+  const int a = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave, and its block row
+  // workgroups spread their atomics over `reps` copies of the accumulator, so
+  // a body pair shared by all is not one chain of atomics per value
   double* out = acc_reps + (blockIdx.x % reps) * rep_stride;
-  const long long w0 = (long long)blockIdx.x * per_wave;
-  if (w0 >= m) return;
-  const long long w1 = w0 + per_wave < m ? w0 + per_wave : m;
-  float acc[144];
+  const long long w0 = (long long)blockIdx.x * per_block;
+  const long long w1 = w0 + per_block < m ? w0 + per_block : m;
+  float acc[36];
 #pragma unroll
-  for (int k = 0; k < 144; ++k) acc[k] = 0.0f;
+  for (int k = 0; k < 36; ++k) acc[k] = 0.0f;
   int cur_a = -1, cur_b = -1;
-  for (long long base = w0; base < w1; base += 64) {
-    const long long t = base + lane;
-    int bi = -1, bj = -1;
-    const bool kept = t < w1 && triplet_pair(rows, cols, vals, int(t), nv, nb, body, fixed, bi, bj);
-    // a lane moving to another body pair first hands its sums to the wave
-    if (__ballot(kept && cur_a >= 0 && (bi != cur_a || bj != cur_b)))
-      flush_pairs(cur_a, cur_b, acc, lane, poff, pcol, sh, out);
-    if (kept) {
-      cur_a = bi;
-      cur_b = bj;
-      const int r = rows[t], c = cols[t];
-      const float ca[4] = {1.0f, rest[3ll * r], rest[3ll * r + 1], rest[3ll * r + 2]};
-      const float cc[4] = {1.0f, rest[3ll * c], rest[3ll * c + 1], rest[3ll * c + 2]};
-      float h[9];
+  int buf = 0;
+  for (long long tile = w0; tile < w1; tile += kQueueTile, buf ^= 1) {
+    bool keep[kQueuePer];
+    int before[kQueuePer];
 #pragma unroll
-      for (int k = 0; k < 9; ++k) h[k] = vals[9 * t + k];
+    for (int k = 0; k < kQueuePer; ++k) {
+      const long long t = tile + k * kB + threadIdx.x;
+      int bi, bj;
+      keep[k] = t < w1 && free_pair(rows[t], cols[t], nv, nb, body, fixed, bi, bj) && any_nonzero(vals + 9 * t);
+    }
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+    for (int k = 0; k < kQueuePer; ++k) {
+      const unsigned long long b = __ballot(keep[k]);
+      before[k] = __popcll(b & ((1ull << lane) - 1));
+      if (lane == 0) num[buf][k * kWaves + a] = __popcll(b);
+    }
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int j = 0; j < kQueuePer * kWaves; ++j) {
+      const int c = num[buf][j];
+      if (j % kWaves == a) before[j / kWaves] += total;
+      total += c;
+    }
+#pragma unroll
+    for (int k = 0; k < kQueuePer; ++k)
+      if (keep[k]) queue[buf][before[k]] = int(tile + k * kB + threadIdx.x);
+    __syncthreads();
+    for (int q = 0; q < total; q += 64) {
+      const bool kept = q + lane < total;
+      const long long t = kept ? queue[buf][q + lane] : 0;
+      int r = 0, c = 0, bi = -1, bj = -1;
+      float h[9], ca = 1.0f, cc[4];
+      if (kept) {
+        r = rows[t];
+        c = cols[t];
+        __builtin_memcpy(h, vals + 9 * t, sizeof(h));
+        bi = body[r];
+        bj = body[c];
+        if (a > 0) ca = rest[3ll * r + a - 1];
+        cc[0] = 1.0f;
+        __builtin_memcpy(cc + 1, rest + 3ll * c, 12);
+      }
+      // a lane moving to another body pair first hands its sums to the wave
+      if (__ballot(kept && cur_a >= 0 && (bi != cur_a || bj != cur_b)))
+        flush_pairs(cur_a, cur_b, acc, lane, a, poff, pcol, sh[a], out);
+      if (kept) {
+        cur_a = bi;
+        cur_b = bj;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
-          const float w = ca[a] * cc[b];
+          const float w = ca * cc[b];
 #pragma unroll
-          for (int k = 0; k < 9; ++k) acc[(a * 4 + b) * 9 + k] += w * h[k];
+          for (int k = 0; k < 9; ++k) acc[b * 9 + k] = fmaf(w, h[k], acc[b * 9 + k]);
         }
+      }
     }
   }
-  flush_pairs(cur_a, cur_b, acc, lane, poff, pcol, sh, out);
+  flush_pairs(cur_a, cur_b, acc, lane, a, poff, pcol, sh[a], out);
+}
+
+// One wave a value, a lane a copy: for few values, whose copies one lane
+// would wait for in turn.
+__global__ void finish_few_kernel(const double* acc, int n, int reps, double scale, float* values) {
+  const int i = (blockIdx.x * kB + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+  if (i >= n) return;
+  double v = lane < reps ? acc[(long long)lane * n + i] : 0.0;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  if (lane == 0) values[i] = static_cast<float>(scale * v);
 }
 
 __global__ void finish_values_kernel(const double* acc, long long n, int reps, double scale, float* values) {
@@ -365,42 +376,60 @@ __global__ void finish_values_kernel(const double* acc, long long n, int reps, d
 }
 
 // Forces: vertex i of a free body adds (f, r.x f, r.y f, r.z f) to its
-// body's four rows; the wave adds its lanes' terms per body.
-__global__ __launch_bounds__(kB) void reduce_force_kernel(const float* force, const float* rest, const int* body,
-                                                          const int* fixed, int nv, int nb, double* out) {
+// body's four rows. A wave walks a run of vertices, a lane adding up while
+// its body stays the same; on a change the wave adds its lanes' terms per
+// body. (One flush for every 64 vertices made 1844 atomics on each of a
+// body's 12 sums, which serialise: 17 us on 118k vertices, 12 now.)
+constexpr int kForceRun = 8;
+__global__ __launch_bounds__(kB) void reduce_force_kernel(const float* __restrict__ force,
+                                                          const float* __restrict__ rest,
+                                                          const int* __restrict__ body,
+                                                          const int* __restrict__ fixed, int nv, int nb, double* out) {
   const int lane = threadIdx.x & 63;
-  const int i = blockIdx.x * kB + threadIdx.x;
-  int b = -1;
+  const long long first = (long long)(blockIdx.x * kWaves + (threadIdx.x >> 6)) * 64 * kForceRun + lane;
+  int cur = -1;
   float v[12];
-  if (i < nv) {
-    b = body[i];
-    if (unsigned(b) >= unsigned(nb) || fixed[b]) b = -1;
-  }
-  if (b >= 0) {
-    const float f[3] = {force[3ll * i], force[3ll * i + 1], force[3ll * i + 2]};
-    const float c[4] = {1.0f, rest[3ll * i], rest[3ll * i + 1], rest[3ll * i + 2]};
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+  for (int k = 0; k < 12; ++k) v[k] = 0.0f;
+  auto flush = [&]() {
+    while (true) {
+      const unsigned long long pend = __ballot(cur >= 0);
+      if (!pend) break;
+      const int B = __shfl(cur, __ffsll(static_cast<long long>(pend)) - 1);
+      const bool mine = cur == B;
+      float keep = 0.0f;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) v[3 * a + k] = c[a] * f[k];
-  } else {
+      for (int k = 0; k < 12; ++k) {
+        const float s = wave_sum(mine ? v[k] : 0.0f);
+        if (lane == k) keep = s;
+      }
+      if (lane < 12) atomicAdd(out + 12ll * B + lane, static_cast<double>(keep));
+      if (mine) {
+        cur = -1;
 #pragma unroll
-    for (int k = 0; k < 12; ++k) v[k] = 0.0f;
-  }
-  while (true) {
-    const unsigned long long pend = __ballot(b >= 0);
-    if (!pend) break;
-    const int B = __shfl(b, __ffsll(static_cast<long long>(pend)) - 1);
-    const bool mine = b == B;
-    float keep = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-      const float s = wave_sum(mine ? v[k] : 0.0f);
-      if (lane == k) keep = s;
+        for (int k = 0; k < 12; ++k) v[k] = 0.0f;
+      }
     }
-    if (lane < 12) atomicAdd(out + 12ll * B + lane, static_cast<double>(keep));
-    if (mine) b = -1;
+  };
+  for (int q = 0; q < kForceRun; ++q) {
+    const long long i = first + 64 * q;
+    int b = -1;
+    if (i < nv) {
+      b = body[i];
+      if (unsigned(b) >= unsigned(nb) || fixed[b]) b = -1;
+    }
+    if (__ballot(b >= 0 && cur >= 0 && b != cur)) flush();
+    if (b >= 0) {
+      cur = b;
+      const float f[3] = {force[3 * i], force[3 * i + 1], force[3 * i + 2]};
+      const float c[4] = {1.0f, rest[3 * i], rest[3 * i + 1], rest[3 * i + 2]};
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v[3 * a + k] = fmaf(c[a], f[k], v[3 * a + k]);
+    }
   }
+  flush();
 }
 
 __global__ void finish_force_kernel(const double* acc, int n, float* out) {
@@ -486,7 +515,7 @@ int ipc_abd_reduce_contacts(ipc_abd* w, int n_bodies, const int* body, const flo
   if (force) {
     e = zero_f64(w->facc.as<double>(), 12ll * nb, s);
     if (e == hipSuccess && n_vertices > 0)
-      hipLaunchKernelGGL(reduce_force_kernel, dim3(nblk(n_vertices, kB)), dim3(kB), 0, s, force, rest, body, fixed,
+      hipLaunchKernelGGL(reduce_force_kernel, dim3(nblk(n_vertices, kB * kForceRun)), dim3(kB), 0, s, force, rest, body, fixed,
                          n_vertices, nb, w->facc.as<double>());
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess)
@@ -498,20 +527,22 @@ int ipc_abd_reduce_contacts(ipc_abd* w, int n_bodies, const int* body, const flo
   if (blocks == 0) return IPC_OK;
   e = zero_f64(w->acc.as<double>(), 9 * blocks * reps, s);
   if (e == hipSuccess && n_triplets > 0) {
-    // each wave a contiguous run of at least 64 triplets, about 4096 waves
-    long long per = (n_triplets + 4095) / 4096;
-    per = (per + 63) / 64 * 64;
-    const long long waves = (n_triplets + per - 1) / per;
-    hipLaunchKernelGGL(reduce_hessian_kernel, dim3(int(waves)), dim3(64), 0, s, rows, cols, vals, n_triplets,
-                       int(per), n_vertices, nb, body, fixed, rest, w->poff.as<int>(), w->pcol.as<int>(),
-                       w->acc.as<double>(), int(reps), 9 * blocks);
+    // each workgroup a contiguous run of whole tiles, about 2048 workgroups
+    const long long per = ((long long)n_triplets + 2048ll * kQueueTile - 1) / (2048ll * kQueueTile) * kQueueTile;
+    hipLaunchKernelGGL(reduce_hessian_kernel, dim3(unsigned((n_triplets + per - 1) / per)), dim3(kB), 0, s, rows, cols,
+                       vals, n_triplets, int(per), n_vertices, nb, body, fixed, rest, w->poff.as<int>(),
+                       w->pcol.as<int>(), w->acc.as<double>(), int(reps), 9 * blocks);
     e = hipGetLastError();
   }
   if (e == hipSuccess) {
     const long long n = 9 * blocks;
-    const int g = nblk(n, kB) < 4096 ? nblk(n, kB) : 4096;
-    hipLaunchKernelGGL(finish_values_kernel, dim3(g), dim3(kB), 0, s, w->acc.as<double>(), n, int(reps), scale,
-                       values);
+    // up to 65536 values a wave each still fits the device at once
+    if (n <= 65536)
+      hipLaunchKernelGGL(finish_few_kernel, dim3(nblk(n, kWaves)), dim3(kB), 0, s, w->acc.as<double>(), int(n),
+                         int(reps), scale, values);
+    else
+      hipLaunchKernelGGL(finish_values_kernel, dim3(nblk(n, kB) < 4096 ? nblk(n, kB) : 4096), dim3(kB), 0, s,
+                         w->acc.as<double>(), n, int(reps), scale, values);
     e = hipGetLastError();
   }
   return abd_hip(e, "abd_reduce_contacts: reduce");

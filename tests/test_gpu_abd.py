@@ -89,3 +89,32 @@ def test_capacity_is_reported_before_any_output(dev, oracle):
     torch.cuda.synchronize()
     assert st > 0 and st % 16 == 0 and int(offsets[-1].item()) == st
     assert not rf.any()
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 70001])
+@pytest.mark.parametrize("nb", [1, 3, 40])
+def test_queue_edges_match_oracle(dev, oracle, n, nb):
+    """Triplet counts around a tile of the reduction's queue (1024), bodies
+    that change from lane to lane, zero blocks, vertices out of range, a fixed
+    body, and more body pairs than the mark kernel's LDS set holds (40^2);
+    the reduction's bars."""
+    rng = np.random.default_rng(n + nb)
+    nv = 500
+    body = np.sort(rng.integers(0, nb, nv)).astype(np.int32)
+    fixed = np.zeros(nb, np.int32)
+    if nb > 1:
+        fixed[nb // 2] = 1
+    rest = rng.normal(size=(nv, 3)).astype(np.float32)
+    rows, cols = rng.integers(-1, nv + 1, (2, n)).astype(np.int32)
+    vals = rng.normal(size=(n, 3, 3)).astype(np.float32)
+    vals[rng.random(n) < 0.3] = 0.0
+    force = rng.normal(size=(nv, 3)).astype(np.float32)
+    M, rf = AbdReducer().reduce(nb, *(torch.from_numpy(a).to(dev) for a in (body, rest, fixed, rows, cols, vals, force)),
+                                scale=0.5)
+    o, c, v, a, rref = oracle.abd_reduce(nb, body, rest, fixed, rows, cols, vals, force, 0.5)
+    nnz = int(o[-1])
+    assert np.array_equal(M.offsets.cpu().numpy(), o)
+    assert np.array_equal(M.columns[:nnz].cpu().numpy(), c)
+    err = np.abs(M.values[:nnz].cpu().numpy().astype(np.float64) - v)
+    assert (err <= 1e-5 * a + 6e-8 * np.abs(v) + 1e-30).all()
+    assert np.abs(rf.cpu().numpy() - rref).max() <= 1e-5 * max(np.abs(rref).max(), 1e-30)
