@@ -11,6 +11,7 @@
 #include <cstdio>
 
 #include "../../include/ipc_warp_amd.h"
+#include "force_table.hpp"
 #include "ipc_kernels.hpp"
 
 namespace ipcd {
@@ -148,36 +149,45 @@ __device__ inline M3 pk1(const M3& F, const Snh& s) {
   return add(scale(distortional, F), scale(volumetric, cof));
 }
 
-// Directional derivative of PK1 at F along dF (fem/snh.py:43-84).
-__device__ inline M3 tangent(const M3& F, const M3& dF, const Snh& s) {
-  const M3 cof = cofactor(F);
-  const float Ic = ddot(F, F);
-  const float Ic1 = Ic + 1.0f;
-  const float dIc = 2.0f * ddot(F, dF);
-  const float distortional = s.mu * (1.0f - 1.0f / Ic1);
-  const float d_distortional = s.mu * dIc / (Ic1 * Ic1);
-  const float dJ = ddot(cof, dF);
-  const float volumetric = s.lam * (det3(F) - s.alpha);
-  float f0[3], f1[3], f2[3], g0[3], g1[3], g2[3];
-  col(F, 0, f0);
-  col(F, 1, f1);
-  col(F, 2, f2);
-  col(dF, 0, g0);
-  col(dF, 1, g1);
-  col(dF, 2, g2);
-  float a[3], b[3], c0[3], c1[3], c2[3];
-  cross3(g1, f2, a);
-  cross3(f1, g2, b);
-  c0[0] = a[0] + b[0]; c0[1] = a[1] + b[1]; c0[2] = a[2] + b[2];
-  cross3(g2, f0, a);
-  cross3(f2, g0, b);
-  c1[0] = a[0] + b[0]; c1[1] = a[1] + b[1]; c1[2] = a[2] + b[2];
-  cross3(g0, f1, a);
-  cross3(f0, g1, b);
-  c2[0] = a[0] + b[0]; c2[1] = a[1] + b[1]; c2[2] = a[2] + b[2];
-  const M3 dcof = from_cols(c0, c1, c2);
-  return add(add(add(scale(distortional, dF), scale(d_distortional, F)), scale(s.lam * dJ, cof)),
-             scale(volumetric, dcof));
+// What a tet's directional derivatives share.
+struct Tangent {
+  M3 F, cof;
+  float Ic1, distortional, volumetric;
+};
+__device__ inline Tangent tangent_of(const M3& F, const Snh& s) {
+  Tangent t;
+  t.F = F;
+  t.cof = cofactor(F);
+  t.Ic1 = ddot(F, F) + 1.0f;
+  t.distortional = s.mu * (1.0f - 1.0f / t.Ic1);
+  t.volumetric = s.lam * (det3(F) - s.alpha);
+  return t;
+}
+
+// Directional derivative of PK1 at F (fem/snh.py:43-84) along a dF whose only
+// nonzero row is row k, g: about half the operations of the dense form, whose
+// other terms add exact zeros. g x b with g = g_c e_k (a column of dF) has
+// components p, q = k + 1, k + 2 (mod 3) only: -g_c b_q and g_c b_p.
+template <int k>
+__device__ inline M3 tangent_row(const Tangent& t, const float g[3], const Snh& s) {
+  constexpr int p = (k + 1) % 3, q = (k + 2) % 3;
+  const float dIc = 2.0f * (t.F.m[k][0] * g[0] + t.F.m[k][1] * g[1] + t.F.m[k][2] * g[2]);
+  const float d_distortional = s.mu * dIc / (t.Ic1 * t.Ic1);
+  const float dJ = t.cof.m[k][0] * g[0] + t.cof.m[k][1] * g[1] + t.cof.m[k][2] * g[2];
+  const float lam_dJ = s.lam * dJ;
+  const float vz = t.volumetric * 0.0f;  // dcof's row k is zero
+  M3 o;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    // column c of dcof: g_a x f_b + f_a x g_b with (a, b) the next two columns
+    const int a = (c + 1) % 3, b = (c + 2) % 3;
+    const float dp = t.F.m[q][a] * g[b] - g[a] * t.F.m[q][b];
+    const float dq = g[a] * t.F.m[p][b] - t.F.m[p][a] * g[b];
+    o.m[k][c] = ((t.distortional * g[c] + d_distortional * t.F.m[k][c]) + lam_dJ * t.cof.m[k][c]) + vz;
+    o.m[p][c] = (d_distortional * t.F.m[p][c] + lam_dJ * t.cof.m[p][c]) + t.volumetric * dp;
+    o.m[q][c] = (d_distortional * t.F.m[q][c] + lam_dJ * t.cof.m[q][c]) + t.volumetric * dq;
+  }
+  return o;
 }
 
 __device__ inline bool tet_ok(const int4 t, int nv) {
@@ -236,14 +246,17 @@ __global__ void tet_rest_kernel(const float* __restrict__ xcs, int nv, const int
   W[e] = fabsf(det) / 6.0f;
 }
 
-// Per wave in LDS: its 32 tets' vertex ids and flags, their forces on the
-// way to b, and one block row (blocks (i, 0..3), 36 floats) of each tet's
-// values on the way to memory.
+constexpr int kTetsPerWave = 32;
+constexpr int kTetsPerBlock = 4 * kTetsPerWave;
+
+// In LDS: per wave its 32 tets' vertex ids and flags and one block row
+// (blocks (i, 0..3), 36 floats) of each tet's values on the way to memory;
+// the workgroup's forces on the way to b.
 struct TetStage {
-  float f[4][32 * 12];
   int v[4][32 * 4];
   int ok[4][32];
   float4 row[4][32 * 9];
+  ForceTable<float, 8 * kTetsPerBlock> force;
 };
 
 // Two lanes per tet, lanes p and p + 32 of a wave: the first takes the
@@ -258,10 +271,12 @@ struct TetStage {
 // row i there), and the wave stores 32 tets' row i with consecutive lanes
 // on consecutive 16-byte words; a lane storing its own tet's 576 bytes
 // touched 64 cache lines per store instruction. Row and column indices go
-// out the same way from the staged vertex ids.
-constexpr int kTetsPerWave = 32;
-constexpr int kTetsPerBlock = 4 * kTetsPerWave;
-
+// out the same way from the staged vertex ids. The forces of the workgroup's
+// 128 tets are summed per vertex in LDS first: of their 512 corners a mesh's
+// neighbouring tets share all but a sixth, and the device atomics on every
+// corner took 32 of the 131 us of 444,528 tets (14 of 106 now). Four lanes a tet
+// (95 registers, five waves a SIMD, not 152 and three) took 111: the shared F and
+// cofactors weigh more than the waves.
 __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restrict__ x, int nv,
                                                           const int4* __restrict__ T, int n,
                                                           const float* __restrict__ Bmv, const float* __restrict__ Wv,
@@ -271,66 +286,58 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int p = lane & 31, half = lane >> 5;
   const int first = blockIdx.x * kTetsPerBlock + wave * kTetsPerWave;
-  if (first >= n) return;  // the whole wave is past the end
-  const int nw = min(kTetsPerWave, n - first);
+  const int nw = first < n ? min(kTetsPerWave, n - first) : 0;  // 0: the whole wave is past the end
   const int e = first + p;
+  force_clear(st.force);
   int4 t = make_int4(0, 0, 0, 0);
   bool ok = false;
   if (e < n) {
     t = T[e];
     ok = tet_ok(t, nv);
   }
+  __syncthreads();
   // h[jj][k][l][i] = dH(j, k).m[l][i] with j = 2 half + jj, i < 3: entry
   // (l, k) of block (i, j)
   float h[2][3][3][3];
-  float force[12];
-#pragma unroll
-  for (int q = 0; q < 12; ++q) force[q] = 0.0f;
   if (ok) {
     const Snh s = reparam(mu, lam);
     M3 Bm;
     const M3 F = deformation(x, t, Bmv + 9ll * e, Bm);
     const float W = Wv[e];
+    const Tangent D = tangent_of(F, s);
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
+    for (int jj = 0; jj < 2; ++jj) {
+      // the nonzero row of dF = dDs Bm: -Bm's row j, and for j = 3 the rows' sum
+      float g[3];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const int j = 2 * half + jj;
-        M3 dDs = mzero();
-        if (j < 3) {
-          dDs.m[k][0] = j == 0 ? -1.0f : 0.0f;
-          dDs.m[k][1] = j == 1 ? -1.0f : 0.0f;
-          dDs.m[k][2] = j == 2 ? -1.0f : 0.0f;
-        } else {
-          dDs.m[k][0] = 1.0f;
-          dDs.m[k][1] = 1.0f;
-          dDs.m[k][2] = 1.0f;
-        }
-        const M3 dF = matmul(dDs, Bm);
-        const M3 dP = tangent(F, dF, s);
+      for (int c = 0; c < 3; ++c)
+        g[c] = jj == 0 ? -(half ? Bm.m[2][c] : Bm.m[0][c])
+                       : (half ? (Bm.m[0][c] + Bm.m[1][c]) + Bm.m[2][c] : -Bm.m[1][c]);
+      auto derivative = [&](const M3& dP, int k) {
         const M3 dH = matmul_t(scale(-W, dP), Bm);
 #pragma unroll
         for (int l = 0; l < 3; ++l)
 #pragma unroll
           for (int i = 0; i < 3; ++i) h[jj][k][l][i] = dH.m[l][i];
-      }
+      };
+      derivative(tangent_row<0>(D, g, s), 0);
+      derivative(tangent_row<1>(D, g, s), 1);
+      derivative(tangent_row<2>(D, g, s), 2);
+    }
     if (b && half == 0) {
       // columns of H = -W P Bm^T, the last the negated sum
       const M3 H = matmul_t(scale(-W, pk1(F, s)), Bm);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int l = 0; l < 3; ++l)
-          force[3 * i + l] = i == 3 ? ((-H.m[l][0]) - H.m[l][1]) - H.m[l][2] : H.m[l][i];
+      force_add(st.force, t.x, H.m[0][0], H.m[1][0], H.m[2][0]);
+      force_add(st.force, t.y, H.m[0][1], H.m[1][1], H.m[2][1]);
+      force_add(st.force, t.z, H.m[0][2], H.m[1][2], H.m[2][2]);
+      force_add(st.force, t.w, ((-H.m[0][0]) - H.m[0][1]) - H.m[0][2], ((-H.m[1][0]) - H.m[1][1]) - H.m[1][2],
+                ((-H.m[2][0]) - H.m[2][1]) - H.m[2][2]);
     }
   }
-  float* sf = st.f[wave];
   int* sv = st.v[wave];
   int* so = st.ok[wave];
   float* sr = reinterpret_cast<float*>(st.row[wave]);
   if (half == 0) {
-#pragma unroll
-    for (int q = 0; q < 12; ++q) sf[p * 12 + q] = force[q];
     sv[p * 4 + 0] = t.x;
     sv[p * 4 + 1] = t.y;
     sv[p * 4 + 2] = t.z;
@@ -378,14 +385,9 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
-  // forces into b, component q of the wave's 12 nw by lane q % 64, so that
-  // one atomic instruction adds consecutive components of consecutive tets
   if (b) {
-    for (int q = lane; q < 12 * nw; q += 64) {
-      const float v = sf[q];
-      const int sl = q / 12, comp = q - 12 * sl, vert = comp / 3;
-      if (so[sl] && v != 0.0f) atomicAdd(b + 3ll * sv[sl * 4 + vert] + (comp - 3 * vert), v);
-    }
+    __syncthreads();
+    force_flush(st.force, b);
   }
 }
 

@@ -68,3 +68,32 @@ def test_out_of_range_tets_write_zeros(dev):
     torch.cuda.synchronize()
     assert W[1].item() == 0.0 and (rows[16:] == 0).all() and (vals[16:] == 0).all()
     assert torch.isfinite(vals[:16]).all()
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 127, 128, 129, 1000])
+def test_partial_workgroups_and_shared_vertices(dev, oracle, n):
+    """Tet counts around a wave's 32 and a workgroup's 128, every tet on its
+    own vertices, tets sharing four vertices, and vertices that collide in the
+    workgroup's force table (1024 apart and more): blocks bit-exact, forces
+    within the rounding of the float sums of at most n terms."""
+    rng = np.random.default_rng(n)
+    unit = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]], np.float32)
+    for kind in ("own", "shared", "apart"):
+        nv = {"own": 4 * n, "shared": 4, "apart": 4096 * 4}[kind]
+        xcs = (np.tile(unit, (nv // 4, 1)) + 0.1 * rng.normal(size=(nv, 3))).astype(np.float32)
+        x = (xcs + 0.1 * rng.normal(size=xcs.shape)).astype(np.float32)
+        first = {"own": 4 * np.arange(n), "shared": np.zeros(n, int), "apart": 1024 * rng.integers(0, 16, n)}[kind]
+        T = (first[:, None] + np.arange(4)).astype(np.int32)
+        xcs_t, x_t, T_t = (torch.from_numpy(a).to(dev) for a in (xcs, x, T))
+        Bm, W = ops.tet_rest(xcs_t, T_t)
+        rows = torch.empty(16 * n, dtype=torch.int32, device=dev)
+        cols = torch.empty_like(rows)
+        vals = torch.empty((16 * n, 3, 3), dtype=torch.float32, device=dev)
+        b = torch.zeros_like(x_t)
+        ops.tet_hessian(x_t, T_t, Bm, W, MU, LAM, rows, cols, vals, b)
+        torch.cuda.synchronize()
+        rBm, rW = oracle.tet_rest(xcs, T)
+        rr, rc, rv, rf = oracle.tet_hessian(x, T, rBm, rW, MU, LAM)
+        assert np.array_equal(rows.cpu().numpy(), rr) and np.array_equal(cols.cpu().numpy(), rc)
+        assert np.array_equal(vals.cpu().numpy().view(np.uint32), rv.view(np.uint32))
+        assert np.abs(b.cpu().numpy() - rf).max() <= max(n, 16) * 2.0 ** -23 * np.abs(rf).max()
