@@ -400,3 +400,27 @@ def test_misaligned_lists_are_refused(dev, oracle):
         assert b"aligned" in lib().ipc_last_error()
     torch.cuda.synchronize()
     assert int(cnt.item()) == -7
+
+
+@pytest.mark.parametrize("n_edges", [1, 2, 7, 4095, 4096, 4097, 12288, 12289])
+def test_queries_per_wave_keep_the_sets(dev, oracle, n_edges):
+    """Edge counts around the changes from two to four and eight queries a
+    wave (and last waves that start with fewer than their share): contacts,
+    candidates and the step bound equal the oracle's."""
+    soup = scenes.two_cubes_on_ground(seed=21, n=19, gap=4e-4, jitter=2e-4)
+    rng = np.random.default_rng(n_edges)
+    soup.edges = np.ascontiguousarray(soup.edges[np.sort(rng.permutation(len(soup.edges))[:n_edges])])
+    S = _solver(dev, soup)
+    _check_dcd(S, soup, False)
+    dx = (2e-3 * rng.standard_normal(soup.x.shape)).astype(np.float32)
+    x1 = S.x - torch.from_numpy(dx).to(dev)
+    for kind, topo in (("ee", soup.edges), ("pt", soup.triangles)):
+        quads, ids = S.ccd_candidates(kind, S.x, x1)
+        fn = oracle.ccd_candidates_ee if kind == "ee" else oracle.ccd_candidates_pt
+        rq, ri = fn(soup.x, x1.cpu().numpy(), topo, soup.body)
+        if len(rq) or len(quads):
+            q, i = _sorted(quads.cpu().numpy(), ids.cpu().numpy())
+            assert np.array_equal(i, ri) and np.array_equal(q, rq)
+    toi = S.raw_toi(torch.from_numpy(dx).to(dev))
+    assert abs(toi - oracle.ccd_toi(soup.x, soup.x - dx, soup.edges, soup.triangles, soup.body, relative=True,
+                                    threads=8)) <= 1e-12
