@@ -97,3 +97,18 @@ def test_features_argument_checks(dev):
         warmstart.vertex_features(x, None, c, 1, c, 0, 0.0)
     with pytest.raises(ValueError):
         warmstart.vertex_features(x, None, c.long(), 1, c, 0, DHAT)
+
+
+@pytest.mark.parametrize("n_ee,n_pt", [(1, 0), (0, 1), (63, 65), (64, 64), (4097, 129)])
+@pytest.mark.parametrize("V", [4, 31, 33])
+def test_features_lane_groups(dev, oracle, n_ee, n_pt, V):
+    """Record counts around a workgroup's 64 (four lanes each), vertex counts
+    around its 32 (eight lanes each), every vertex in far more records than
+    its six slots hold, and no base values."""
+    rng = np.random.default_rng(n_ee + V)
+    x = rng.normal(size=(V, 3)).astype(np.float32)
+    ee, pt = (np.stack([rng.permutation(V)[:4] for _ in range(n)]).astype(np.int32).reshape(-1, 4) if n else
+              np.zeros((0, 4), np.int32) for n in (n_ee, n_pt))
+    ref = oracle.warmstart_features(x, None, ee, pt, DHAT)
+    got = _gpu(dev, x, None, ee, pt)
+    assert np.array_equal(got.view(np.uint32), np.asarray(ref, np.float32).view(np.uint32))
