@@ -112,7 +112,9 @@ __device__ inline void atomic_min_scalar(double* p, double v) {
 }
 
 // accumulate_vertex_toi (augmented_lagrangian.py:105-113); vertices out of
-// range are skipped.
+// range are skipped. A plain load first, to pass an atomic that cannot lower the
+// value, costs more than the atomics that it saves (96,691 records of 96,691
+// vertices: 19 us with it, 11.5 without).
 template <typename S>
 __global__ __launch_bounds__(kB) void vertex_toi_kernel(const unsigned* rec, int n, S* vertex_toi, int nv) {
   using L = Layout<S>;
@@ -204,8 +206,10 @@ __global__ __launch_bounds__(kB) void scatter_kernel(const int* bucket, int m, c
 
 // Slot s of [0, capacity): below the entry count, the input in slot s goes
 // to start[b] + (inputs of its bucket with a larger index); the slots past
-// the count are zeroed. The 256 records of a workgroup are then written one
-// word per lane. CREATE builds fresh entries from XConstraint records
+// the count are zeroed. The 256 records of a workgroup are then written two
+// words per lane, a batch of loads in flight before its stores (a word at a
+// time, each load waited for the store before it: 131,072 slots 15.2 us,
+// 8.0 now). CREATE builds fresh entries from XConstraint records
 // (to_al_constraint, augmented_lagrangian.py:88-102); otherwise entries
 // are copied whole from the old ([0, n_old)) or the new table.
 template <typename S, bool CREATE>
@@ -213,6 +217,8 @@ __global__ __launch_bounds__(kB) void gather_kernel(const unsigned* in_a, int n_
                                                     const int* src, const int* bucket, const int* start,
                                                     int table_size, int capacity, unsigned* out) {
   using L = Layout<S>;
+  constexpr int kBatch = (L::kAWords / 2 + 1) / 2;
+  static_assert(L::kAWords % 2 == 0 && L::kCopied % 2 == 0, "records in pairs of words");
   __shared__ const unsigned* rec_src[kB];
   __shared__ int rec_dst[kB];
   const int total = start[table_size];
@@ -239,18 +245,28 @@ __global__ __launch_bounds__(kB) void gather_kernel(const unsigned* in_a, int n_
   }
   __syncthreads();
   const int nrec = min(kB, capacity - base);
-  for (int f = threadIdx.x; f < nrec * L::kAWords; f += kB) {
-    const int r = f / L::kAWords;
-    const int w = f - r * L::kAWords;
-    const unsigned* p = rec_src[r];
-    unsigned v = 0u;
-    if (p) {
+#pragma unroll 1
+  for (int k0 = 0; k0 < L::kAWords / 2; k0 += kBatch) {
+    uint2 v[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const int f = (k0 + k) * kB + threadIdx.x;
+      const int r = f / (L::kAWords / 2), w = 2 * (f - r * (L::kAWords / 2));
+      v[k] = make_uint2(0u, 0u);
+      if (r >= nrec) continue;
+      const unsigned* p = rec_src[r];
+      if (!p) continue;
       if (!CREATE || w < L::kCopied)
-        v = p[w];
-      else if (w == L::kGammaWord + L::kSw - 1 || w == L::kMollifierWord + L::kSw - 1)
-        v = L::kOneHi;  // gamma = mollifier = 1; lam, slack, type, d0, grad = 0
+        __builtin_memcpy(&v[k], p + w, sizeof(uint2));
+      else if (w == L::kGammaWord - (L::kSw == 1) || w == L::kMollifierWord - (L::kSw == 1))
+        v[k].y = L::kOneHi;  // gamma = mollifier = 1; lam, slack, type, d0, grad = 0
     }
-    out[static_cast<long long>(rec_dst[r]) * L::kAWords + w] = v;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const int f = (k0 + k) * kB + threadIdx.x;
+      const int r = f / (L::kAWords / 2), w = 2 * (f - r * (L::kAWords / 2));
+      if (r < nrec) __builtin_memcpy(out + static_cast<long long>(rec_dst[r]) * L::kAWords + w, &v[k], sizeof(uint2));
+    }
   }
 }
 

@@ -77,18 +77,23 @@ __global__ __launch_bounds__(kScanB) void scan_tiles_kernel(const int* in, int n
 
 // Adds to each tile past the first what the tiles before it sum to; every
 // workgroup adds those sums itself (there are few), which saves the launch
-// of a scan of theirs.
-__global__ void scan_add_kernel(int* out, int n, const int* tile_sum) {
+// of a scan of theirs. The tile is read whole before any of it is written:
+// read and written a value at a time, the sixteen accesses of a lane waited
+// for each other (262k ints, 64 tiles: 6.5 us, 4.5 now).
+__global__ __launch_bounds__(kScanB) void scan_add_kernel(int* out, int n, const int* tile_sum) {
   __shared__ int sh[4];
   const int tile = blockIdx.x + 1;
+  const long long base = (long long)tile * kScanTile + threadIdx.x;
+  int v[kScanPer];
+#pragma unroll
+  for (int k = 0; k < kScanPer; ++k) v[k] = base + k * kScanB < n ? out[base + k * kScanB] : 0;
   int part = 0;
   for (int i = threadIdx.x; i < tile; i += kScanB) part += tile_sum[i];
   int add;
   block_exclusive(part, sh, add);
-  const long long base = (long long)tile * kScanTile + threadIdx.x;
 #pragma unroll
   for (int k = 0; k < kScanPer; ++k)
-    if (base + k * kScanB < n) out[base + k * kScanB] += add;
+    if (base + k * kScanB < n) out[base + k * kScanB] = v[k] + add;
 }
 
 // out[0..n) = exclusive prefix sums of in[0..n); in and out distinct. `part`

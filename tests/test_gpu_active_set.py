@@ -244,3 +244,20 @@ def test_refused_arguments(dev):
     assert L.ipc_al_merge(A._ws.handle, 104, h.cell_start.data_ptr(), h.cell_entries.data_ptr(), h.table_size, 3,
                           h.cell_entries.data_ptr(), 3, h.table_size, None, None, 4, s) == IPC_EINVAL
     assert L.ipc_al_vertex_toi(r.data_ptr(), 44, 8, vt.data_ptr(), 4, s) == IPC_EINVAL
+
+
+@pytest.mark.parametrize("scalar", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n,cap", [(1, 1), (255, 255), (256, 257), (257, 511), (513, 1024)])
+def test_gather_workgroup_edges(dev, oracle, scalar, n, cap):
+    """Slots around a workgroup's 256 (written two words a lane, in batches):
+    full, one short, one over, and a zeroed tail of its own workgroups."""
+    rng = np.random.default_rng(n)
+    words = random_records(rng, n, 4 * n + 4, scalar)
+    check_against_oracle(oracle, dev, words, 4 * n + 4, scalar, 2 * cap, cap)
+
+
+@pytest.mark.parametrize("T", [4094, 4095, 4096, 8191, 8192, 70001])
+def test_scan_tile_edges(dev, oracle, T):
+    """Bucket counts T + 1 around the scan's tiles of 4096."""
+    rng = np.random.default_rng(T)
+    check_against_oracle(oracle, dev, random_records(rng, 900, 300, torch.float32), 300, torch.float32, T, 1024)
