@@ -5,6 +5,7 @@
 // (16 B, one 128-bit load per lane, coalesced across the wave). Vertex
 // positions are gathered from the float32 [V, 3] array (L2/MALL resident at
 // every configuration this library targets).
+#include "force_sums.hpp"
 #include "ipc_device.hpp"
 #include "ipc_kernels.hpp"
 
@@ -150,28 +151,88 @@ struct HessianArgsT {
 };
 using HessianArgs = HessianArgsT<float, float>;
 
-// Per wave in LDS: the forces on their way to b (12 per contact slot), the
-// slots' 4 vertex ids and active flags, and 144 bytes of every slot's
-// triplet values on their way to memory (one block row in fp32, half of one
-// in fp64).
+// Per wave in LDS: the slots' 4 vertex ids (0 for an inactive contact); the
+// forces; and the triplet values on their way to memory.
+//
+// fp32: `c` holds every slot's compressed Hessian, kField floats each (the
+// fields at the offsets below; 52 = 20 mod 32 lets eight slots' 16-byte
+// reads fall on all banks), and `out` the values of eight contacts a wave.
+// fp64: `out` holds half of one block row (144 bytes) of every slot.
+constexpr int kField = 52;
+enum { kFr = 0, kFcn = 3, kFNtt = 4, kFcg = 10, kFwhat = 12, kFw = 16, kFu = 20, kFs = 36 };
+template <typename R>
+struct ValueStageT;
+template <>
+struct ValueStageT<float> {
+  float c[64 * kField];
+  float4 out[8 * 36];
+};
+template <>
+struct ValueStageT<double> {
+  float4 out[64 * 9];
+};
 template <typename R>
 struct HessianStageT {
-  R f[4][64 * 12];
+  union {
+    ForceSums<R, 4> force;
+    R f[64 * 12];
+    ValueStageT<R> val;
+  } u[4];
   int v[4][64 * 4];
-  int act[4][64];
-  float4 row[4][64 * 9];
 };
 
-// The wave's triplets are one contiguous range of memory (16 blocks per
-// contact, its contacts consecutive). A lane computes its own contact, but
-// the stores are issued for consecutive addresses across the wave: a lane
-// writing its own contact's 576 contiguous bytes made every store
-// instruction touch 64 cache lines with 16 bytes each, and those stores
-// took about half of the kernel's time. Row and column indices are stored
-// from the staged vertex ids; the values go block row by block row through
-// LDS (each lane expands its contact's row q, then the wave stores the 64
-// contacts' rows q, 144 contiguous bytes per contact; in fp64 a row goes in
-// two halves of 144 bytes).
+// The wave's triplet values, 576 bytes a contact and its contacts
+// consecutive, written eight contacts (4,608 contiguous bytes) at a time: a
+// lane expands two blocks of one block row, from fields that the eight lanes
+// of a contact read from LDS. Writing the 64 contacts' block rows one after
+// another (144 of every 576 bytes a pass) was bound by lines that left L2
+// before their other parts arrived: 600k records 143 us, 155 with three
+// waves a SIMD in place of two, 134 with two block rows a pass; 108 so.
+__device__ __forceinline__ void write_values(const float* sc, float4* so, float* vals, int nw) {
+  const int i = (threadIdx.x >> 1) & 3, h = threadIdx.x & 1, lane = threadIdx.x & 63;
+  float4* __restrict__ v4 = reinterpret_cast<float4*>(vals);
+#pragma unroll 1
+  for (int s0 = 0; s0 < nw; s0 += 8) {
+    const float* c = sc + (s0 + (lane >> 3)) * kField;
+    float r[4], N[8], ui[4], uj[8], whj[2], wj[2], sj[2];
+    __builtin_memcpy(r, c + kFr, 16);       // r, cn
+    __builtin_memcpy(N, c + kFNtt, 32);     // Ntt, cg
+    __builtin_memcpy(ui, c + kFu + 4 * i, 16);
+    __builtin_memcpy(uj, c + kFu + 8 * h, 32);
+    __builtin_memcpy(whj, c + kFwhat + 2 * h, 8);
+    __builtin_memcpy(wj, c + kFw + 2 * h, 8);
+    __builtin_memcpy(sj, c + kFs + 4 * i + 2 * h, 8);
+    const float cn = r[3], cg = N[6], pi = cn * c[kFwhat + i], gw = cg * c[kFw + i];
+    float o[18];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma clang fp contract(fast)
+      const float rr = gw * wj[k] + cn * sj[k];
+      expand_parts(rr, pi, cn * whj[k], whj[k], r, N, ui, uj + 4 * k, o + 9 * k);
+    }
+    float* p = reinterpret_cast<float*>(so) + lane * 18;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) __builtin_memcpy(p + 2 * k, o + 2 * k, 8);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int m = min(8, nw - s0) * 36;
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+      if (lane + 64 * k < m) v4[s0 * 36 + lane + 64 * k] = so[lane + 64 * k];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+}
+
+// One contact list's block of a launch. The wave's triplets are one
+// contiguous range of memory (16 blocks per contact, its contacts
+// consecutive). A lane computes its own contact, but the stores are issued
+// for consecutive addresses across the wave: a lane writing its own
+// contact's 576 contiguous bytes made every store instruction touch 64 cache
+// lines with 16 bytes each, and those stores took about half of the kernel's
+// time. Row and column indices are stored from the staged vertex ids. The
+// fp64 values go through LDS in eight passes, each lane expanding half of a
+// block row of its contact (144 bytes) before the wave stores the halves:
+// there the arithmetic is the bound (150k records 102 us, 100 without any
+// store).
 template <bool EE, typename P, typename R>
 __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int block, HessianStageT<R>& st) {
   const P* __restrict__ x = A.x;
@@ -183,8 +244,6 @@ __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int b
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = contact_slot(lpw, block);
   R force[12];
-#pragma unroll
-  for (int k = 0; k < 12; ++k) force[k] = R(0);
   int4 c = make_int4(0, 0, 0, 0);
   CompressedHessianT<R> C;
   bool active = false;
@@ -193,22 +252,71 @@ __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int b
     active = valid4(c, nv) && (EE ? pair_ee<P, R>(x, xcs, c, l0, kappa, true, C, force, nullptr)
                                   : pair_pt<P, R>(x, c, l0, kappa, true, C, force, nullptr));
   }
-  if (!active) {
+  // Forces into b. Device-scope float atomics cost a transaction per cache
+  // line that an instruction touches. A full wave sums its contacts' forces
+  // per vertex first: contacts that lie close share vertices (911k of a rod
+  // twist: 2.8M lines, 0.48M so, and the kernel 237 and 169 us; 600k that share
+  // none: 108 and 125). The sparse waves of a short list take the
+  // work of a full one for a quarter of the contacts (150k in fp64: 110 us,
+  // 104 without), and add their force components transposed from LDS, value
+  // j by lane j % 64, so that an instruction touches a few lines where
+  // vertices are adjacent.
+  if (lpw == 64) {
+    const int verts[4] = {c.x, c.y, c.z, c.w};
+    add_forces(st.u[wave].force, verts, force, active, b);
+  } else {
+    R* sf = st.u[wave].f;
+    int* sv = st.v[wave];
+    if (lane < lpw) {
 #pragma unroll
-    for (int k = 0; k < 12; ++k) force[k] = R(0);
+      for (int k = 0; k < 12; ++k) sf[lane * 12 + k] = active ? force[k] : R(0);
+      sv[lane * 4 + 0] = c.x;
+      sv[lane * 4 + 1] = c.y;
+      sv[lane * 4 + 2] = c.z;
+      sv[lane * 4 + 3] = c.w;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int j = lane; j < 12 * lpw; j += 64) {
+      const R v = sf[j];
+      if (v != R(0)) {
+        const int slot = j / 12, comp = j - 12 * slot, vert = comp / 3;
+        unsafeAtomicAdd(b + 3 * (long long)sv[slot * 4 + vert] + (comp - 3 * vert), v);
+      }
+    }
   }
-  R* sf = st.f[wave];
+  if (!active) c = make_int4(0, 0, 0, 0);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the values take the forces' place
   int* sv = st.v[wave];
-  int* sa = st.act[wave];
-  float4* sr = st.row[wave];
+  ValueStageT<R>& val = st.u[wave].val;
   if (lane < lpw) {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) sf[lane * 12 + k] = force[k];
     sv[lane * 4 + 0] = c.x;
     sv[lane * 4 + 1] = c.y;
     sv[lane * 4 + 2] = c.z;
     sv[lane * 4 + 3] = c.w;
-    sa[lane] = active ? 1 : 0;
+    if constexpr (sizeof(R) == 4) {
+      float t[kField];
+#pragma unroll
+      for (int k = 0; k < kField; ++k) t[k] = 0.0f;
+      if (active) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) t[kFr + k] = C.rh[k];
+        t[kFcn] = C.cn;
+        t[kFcg] = C.cg;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) t[kFNtt + k] = C.Ntt[k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          t[kFwhat + k] = C.what[k];
+          t[kFw + k] = C.w[k];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) t[kFu + 4 * k + a] = C.u[k][a];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) t[kFs + 4 * k + j] = C.s[sidx(k, j)];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kField / 4; ++k) __builtin_memcpy(&val.c[lane * kField + 4 * k], t + 4 * k, 16);
+    }
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   // the wave's contacts [first, first + nw) own triplets [offset + first, ...) * 16
@@ -221,56 +329,38 @@ __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int b
     int4* cols4 = reinterpret_cast<int4*>(A.cols + tbase);
     for (int t = lane; t < nw * 4; t += 64) {
       const int s = t >> 2, ii = t & 3;
-      int4 rv = make_int4(0, 0, 0, 0), cv = make_int4(0, 0, 0, 0);
-      if (sa[s]) {
-        const int vi = sv[s * 4 + ii];
-        rv = make_int4(vi, vi, vi, vi);
-        cv = make_int4(sv[s * 4 + 0], sv[s * 4 + 1], sv[s * 4 + 2], sv[s * 4 + 3]);
-      }
-      rows4[t] = rv;
-      cols4[t] = cv;
+      const int vi = sv[s * 4 + ii];
+      rows4[t] = make_int4(vi, vi, vi, vi);
+      cols4[t] = make_int4(sv[s * 4 + 0], sv[s * 4 + 1], sv[s * 4 + 2], sv[s * 4 + 3]);
     }
   }
-  // values, 144 bytes at a time: kPer consecutive 3x3 blocks of a block row
-  // (4 in fp32, 2 in fp64) = 9 16-byte units; a contact holds 36 kHalves
-  // units, kHalves per block row.
-  constexpr int kHalves = int(sizeof(R)) / 4;
-  constexpr int kPer = 4 / kHalves;
-  float4* v4 = reinterpret_cast<float4*>(A.vals + tbase * 9);
+  if constexpr (sizeof(R) == 4) {
+    write_values(val.c, val.out, A.vals + tbase * 9, nw);
+  } else {
+    // values, 144 bytes at a time: two 3x3 blocks of a block row = 9 16-byte
+    // units; a contact holds 72 units
+    float4* v4 = reinterpret_cast<float4*>(A.vals + tbase * 9);
 #pragma unroll
-  for (int q = 0; q < 4 * kHalves; ++q) {
-    if (lane < lpw) {
-      R blk[9 * kPer];
-      if (active) {
+    for (int q = 0; q < 8; ++q) {
+      if (lane < lpw) {
+        R blk[18];
+        if (active) {
 #pragma unroll
-        for (int r = 0; r < kPer; ++r) expand_block(C, q / kHalves, (q % kHalves) * kPer + r, blk + 9 * r);
-      } else {
+          for (int r = 0; r < 2; ++r) expand_block(C, q / 2, (q % 2) * 2 + r, blk + 9 * r);
+        } else {
 #pragma unroll
-        for (int k = 0; k < 9 * kPer; ++k) blk[k] = R(0);
+          for (int k = 0; k < 18; ++k) blk[k] = R(0);
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) __builtin_memcpy(&val.out[lane * 9 + k], blk + 2 * k, 16);
       }
-#pragma unroll
-      for (int k = 0; k < 9; ++k) __builtin_memcpy(&sr[lane * 9 + k], blk + k * (16 / int(sizeof(R))), 16);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // slot s's part q: unit s * 36 kHalves + q * 9 + k of the wave's range
-    for (int t = lane; t < nw * 9; t += 64) {
-      const int s = t / 9, k = t - 9 * s;
-      v4[s * 36 * kHalves + q * 9 + k] = sr[t];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  }
-  // Forces into b. Device-scope float atomics cost a memory transaction per
-  // cache line an atomic instruction touches. The wave's 12 lpw force
-  // components (contact slot j / 12, component j % 12) are added transposed
-  // from LDS, value j by lane j % 64: an instruction then adds consecutive
-  // components of consecutive contacts, a few lines when their vertices are
-  // adjacent instead of one line per lane. A zero force (a vertex with zero
-  // weight in the contact's feature, or no active contact) is not added.
-  for (int j = lane; j < 12 * lpw; j += 64) {
-    const R v = sf[j];
-    if (v != R(0)) {
-      const int slot = j / 12, comp = j - 12 * slot, vert = comp / 3;
-      unsafeAtomicAdd(b + 3 * (long long)sv[slot * 4 + vert] + (comp - 3 * vert), v);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      // slot s's part q: unit s * 72 + q * 9 + k of the wave's range
+      for (int t = lane; t < nw * 9; t += 64) {
+        const int s = t / 9, k = t - 9 * s;
+        v4[s * 72 + q * 9 + k] = val.out[t];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
   }
 }

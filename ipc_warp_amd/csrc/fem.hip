@@ -11,7 +11,7 @@
 #include <cstdio>
 
 #include "../../include/ipc_warp_amd.h"
-#include "force_table.hpp"
+#include "force_sums.hpp"
 #include "ipc_kernels.hpp"
 
 namespace ipcd {
@@ -249,14 +249,16 @@ __global__ void tet_rest_kernel(const float* __restrict__ xcs, int nv, const int
 constexpr int kTetsPerWave = 32;
 constexpr int kTetsPerBlock = 4 * kTetsPerWave;
 
-// In LDS: per wave its 32 tets' vertex ids and flags and one block row
-// (blocks (i, 0..3), 36 floats) of each tet's values on the way to memory;
-// the workgroup's forces on the way to b.
+// Per wave in LDS: its 32 tets' vertex ids and flags; the forces on the way
+// to b, and then one block row (blocks (i, 0..3), 36 floats) of each tet's
+// values on the way to memory.
 struct TetStage {
   int v[4][32 * 4];
   int ok[4][32];
-  float4 row[4][32 * 9];
-  ForceTable<float, 8 * kTetsPerBlock> force;
+  union {
+    ForceSums<float, 2> force;
+    float4 row[32 * 9];
+  } u[4];
 };
 
 // Two lanes per tet, lanes p and p + 32 of a wave: the first takes the
@@ -271,10 +273,10 @@ struct TetStage {
 // row i there), and the wave stores 32 tets' row i with consecutive lanes
 // on consecutive 16-byte words; a lane storing its own tet's 576 bytes
 // touched 64 cache lines per store instruction. Row and column indices go
-// out the same way from the staged vertex ids. The forces of the workgroup's
-// 128 tets are summed per vertex in LDS first: of their 512 corners a mesh's
-// neighbouring tets share all but a sixth, and the device atomics on every
-// corner took 32 of the 131 us of 444,528 tets (14 of 106 now). Four lanes a tet
+// out the same way from the staged vertex ids. The forces are
+// summed per vertex over the wave's 32 tets first (neighbouring tets share
+// vertices, and the device atomics on every corner took 32 of the 131 us of
+// 444,528 tets; 97 with float atomics on a table in LDS, 78 so). Four lanes a tet
 // (95 registers, five waves a SIMD, not 152 and three) took 111: the shared F and
 // cofactors weigh more than the waves.
 __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restrict__ x, int nv,
@@ -288,17 +290,16 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
   const int first = blockIdx.x * kTetsPerBlock + wave * kTetsPerWave;
   const int nw = first < n ? min(kTetsPerWave, n - first) : 0;  // 0: the whole wave is past the end
   const int e = first + p;
-  force_clear(st.force);
   int4 t = make_int4(0, 0, 0, 0);
   bool ok = false;
   if (e < n) {
     t = T[e];
     ok = tet_ok(t, nv);
   }
-  __syncthreads();
   // h[jj][k][l][i] = dH(j, k).m[l][i] with j = 2 half + jj, i < 3: entry
   // (l, k) of block (i, j)
   float h[2][3][3][3];
+  float f[12] = {};
   if (ok) {
     const Snh s = reparam(mu, lam);
     M3 Bm;
@@ -327,16 +328,29 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
     if (b && half == 0) {
       // columns of H = -W P Bm^T, the last the negated sum
       const M3 H = matmul_t(scale(-W, pk1(F, s)), Bm);
-      force_add(st.force, t.x, H.m[0][0], H.m[1][0], H.m[2][0]);
-      force_add(st.force, t.y, H.m[0][1], H.m[1][1], H.m[2][1]);
-      force_add(st.force, t.z, H.m[0][2], H.m[1][2], H.m[2][2]);
-      force_add(st.force, t.w, ((-H.m[0][0]) - H.m[0][1]) - H.m[0][2], ((-H.m[1][0]) - H.m[1][1]) - H.m[1][2],
-                ((-H.m[2][0]) - H.m[2][1]) - H.m[2][2]);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) f[3 * c + r] = H.m[r][c];
+        f[9 + c] = ((-H.m[c][0]) - H.m[c][1]) - H.m[c][2];
+      }
     }
+  }
+  if (b) {
+    // the second lane of a tet takes over its last two vertices
+    float g[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      const float u = __shfl(f[6 + q], p, 64);
+      g[q] = half ? u : f[q];
+    }
+    const int verts[2] = {half ? t.z : t.x, half ? t.w : t.y};
+    add_forces(st.u[wave].force, verts, g, ok, b);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the rows take the forces' place
   }
   int* sv = st.v[wave];
   int* so = st.ok[wave];
-  float* sr = reinterpret_cast<float*>(st.row[wave]);
+  float* sr = reinterpret_cast<float*>(st.u[wave].row);
   if (half == 0) {
     sv[p * 4 + 0] = t.x;
     sv[p * 4 + 1] = t.y;
@@ -362,7 +376,7 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
     }
   }
   float4* v4 = reinterpret_cast<float4*>(vals + 9 * t0);
-  const float4* sr4 = st.row[wave];
+  const float4* sr4 = st.u[wave].row;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float blk[18];  // blocks (i, 2 half), (i, 2 half + 1): entry (l, k) of block jj at 9 jj + 3 l + k
@@ -384,10 +398,6 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
       v4[sl * 36 + i * 9 + u] = sr4[q];
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  }
-  if (b) {
-    __syncthreads();
-    force_flush(st.force, b);
   }
 }
 

@@ -589,29 +589,35 @@ IPCD_FN double nsd_compressed(const FeatureGeom& g, bool want_nsd, CompressedHes
   return d2;
 }
 
-// Block (i, j) of the compressed Hessian, row-major 3x3.
+// Block (i, j) of the compressed Hessian, row-major 3x3, from the fields it
+// takes: rr = cg w_i w_j + c_n s_ij, pi = c_n w^_i, whj = w^_j, pj = c_n w^_j.
 template <typename R>
-IPCD_FN void expand_block(const CompressedHessianT<R>& C, int i, int j, R out[9]) {
+IPCD_FN void expand_parts(R rr, R pi, R pj, R whj, const R r[3], const R Ntt[6], const R ui[3], const R uj[3],
+                          R out[9]) {
 #pragma clang fp contract(fast)
   // H_ij[a][b] = c_n w^_i w^_j Ntt[a][b] + r[b] (c_n w^_i u_j[a])
   //            + r[a] (c_n w^_j u_i[b] + rr r[b]): per block three 3-vectors
   //            and the six distinct scaled Ntt entries, then two FMAs an entry.
-  const R rr = C.cg * C.w[i] * C.w[j] + C.cn * C.s[sidx(i, j)];
-  const R* r = C.rh;
-  const R pi = C.cn * C.what[i], pj = C.cn * C.what[j];
-  const R cw = pi * C.what[j];
+  const R cw = pi * whj;
   R A[3], B[3], N[6];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) A[a] = pi * C.u[j][a];
+  for (int a = 0; a < 3; ++a) A[a] = pi * uj[a];
 #pragma unroll
-  for (int b = 0; b < 3; ++b) B[b] = pj * C.u[i][b] + rr * r[b];
+  for (int b = 0; b < 3; ++b) B[b] = pj * ui[b] + rr * r[b];
 #pragma unroll
-  for (int k = 0; k < 6; ++k) N[k] = cw * C.Ntt[k];
+  for (int k = 0; k < 6; ++k) N[k] = cw * Ntt[k];
   const R Nt[9] = {N[0], N[1], N[2], N[1], N[3], N[4], N[2], N[4], N[5]};
 #pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
     for (int b = 0; b < 3; ++b) out[a * 3 + b] = Nt[a * 3 + b] + r[b] * A[a] + r[a] * B[b];
+}
+
+template <typename R>
+IPCD_FN void expand_block(const CompressedHessianT<R>& C, int i, int j, R out[9]) {
+#pragma clang fp contract(fast)
+  const R rr = C.cg * C.w[i] * C.w[j] + C.cn * C.s[sidx(i, j)];
+  expand_parts(rr, C.cn * C.what[i], C.cn * C.what[j], C.what[j], C.rh, C.Ntt, C.u[i], C.u[j], out);
 }
 
 }  // namespace ipcd

@@ -203,3 +203,39 @@ def test_zero_contacts_is_a_noop(dev):
     ops.contact_energy_pt(x, c, 0, L0, KAPPA, e)
     torch.cuda.synchronize()
     assert e.item() == 0.0
+
+
+@pytest.mark.parametrize("kind", ["pt", "ee"])
+@pytest.mark.parametrize("distinct", [1, 5, 40])
+def test_long_list_sums_shared_vertices(dev, oracle, kind, distinct):
+    """Full waves (2^18 contacts and more) whose contacts name few vertices:
+    runs of every length in a wave's sorted forces, across its chunks of 64
+    too, and a last wave that is not full."""
+    n = (1 << 18) + 37
+    x, base = scenes.pair_stream(kind, distinct, seed=distinct)
+    idx = np.random.default_rng(distinct).integers(0, distinct, n)
+    xt = torch.from_numpy(x).to(dev)
+    rows = torch.full((16 * n,), -7, dtype=torch.int32, device=dev)
+    cols = torch.full_like(rows, -7)
+    vals = torch.full((16 * n, 3, 3), float("nan"), dtype=torch.float32, device=dev)
+    b = torch.zeros_like(xt)
+    ct = torch.from_numpy(base[idx]).to(dev)
+    if kind == "ee":
+        ops.contact_hessian_ee(xt, xt, ct, n, L0, KAPPA, rows, cols, vals, b, 0)
+    else:
+        ops.contact_hessian_pt(xt, ct, n, L0, KAPPA, rows, cols, vals, b, 0)
+    r_rows, r_cols, r_vals, r_b, act = oracle.contact_hessian(kind, x, base, L0, KAPPA, threads=8)
+    it = torch.from_numpy(idx).to(dev)
+    for got, want in ((rows, r_rows), (cols, r_cols)):
+        assert torch.equal(got.view(n, 16), torch.from_numpy(want).to(dev).view(distinct, 16)[it])
+    want = torch.from_numpy(r_vals.reshape(distinct, 144)).to(dev)
+    scale = want.abs().amax(1).clamp_min(1e-30)
+    assert (((vals.view(n, 144) - want[it]).abs().amax(1) / scale[it]) <= TOL).all()
+    # a pair's vertices are its own: each takes its force once per repetition.
+    # A wave's sum has 64 terms, and at most one partial sum a wave is added to
+    # another in fp32.
+    times = np.zeros(x.shape[0])
+    times[base] = np.bincount(idx, minlength=distinct)[:, None]
+    f = r_b * times[:, None]
+    bound = (TOL + (n / 64 + 64) * 2.0 ** -24) * np.abs(f).max()
+    assert np.abs(b.cpu().numpy() - f).max() <= bound

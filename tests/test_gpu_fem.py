@@ -97,3 +97,24 @@ def test_partial_workgroups_and_shared_vertices(dev, oracle, n):
         assert np.array_equal(rows.cpu().numpy(), rr) and np.array_equal(cols.cpu().numpy(), rc)
         assert np.array_equal(vals.cpu().numpy().view(np.uint32), rv.view(np.uint32))
         assert np.abs(b.cpu().numpy() - rf).max() <= max(n, 16) * 2.0 ** -23 * np.abs(rf).max()
+
+
+@pytest.mark.parametrize("V,n", [(4, 1), (4, 33), (8, 32), (40, 32), (40, 131), (3000, 257)])
+def test_forces_of_crowded_vertices(dev, oracle, V, n):
+    """Forces summed per vertex over a wave's 32 tets: one tet, four vertices
+    in all of them, runs across the chunks of 64, and hardly any shared."""
+    rng = np.random.default_rng(V + n)
+    xcs, x = rng.random((V, 3)).astype(np.float32), rng.random((V, 3)).astype(np.float32)
+    T = np.stack([rng.permutation(V)[:4] for _ in range(n)]).astype(np.int32)
+    xcs_t, x_t, T_t = (torch.from_numpy(a).to(dev) for a in (xcs, x, T))
+    Bm, W = ops.tet_rest(xcs_t, T_t)
+    rows = torch.empty(16 * n, dtype=torch.int32, device=dev)
+    cols = torch.empty_like(rows)
+    vals = torch.empty((16 * n, 3, 3), dtype=torch.float32, device=dev)
+    b = torch.zeros_like(x_t)
+    ops.tet_hessian(x_t, T_t, Bm, W, MU, LAM, rows, cols, vals, b)
+    rBm, rW = oracle.tet_rest(xcs, T)
+    f = [oracle.tet_hessian(x, T[e:e + 1], rBm[e:e + 1], rW[e:e + 1], MU, LAM)[3] for e in range(n)]
+    # n terms at most a vertex, in any order
+    bound = (n + 1) * 2.0 ** -24 * np.abs(np.asarray(f, np.float64)).sum(0).max()
+    assert np.abs(b.cpu().numpy() - np.asarray(f, np.float64).sum(0)).max() <= bound
