@@ -200,9 +200,14 @@ class ActiveSet:
               "al_create_hash")
 
     def merge(self, new: "ActiveSet") -> None:
-        n_old = self.count()
-        n_new = new.count()
-        destination = self.reserve(max(1, n_old + n_new))
+        # both counts in one copy; the kernels write every word of the
+        # destination, so it is not cleared
+        n_old, n_new = torch.stack((self.hash.cell_start[-1], new.hash.cell_start[-1])).tolist()
+        volume = max(1, n_old + n_new)
+        table_size = max(2, 2 * volume)
+        destination = Hash(table_size, torch.empty(table_size + 1, dtype=torch.int32, device=self.device),
+                           torch.empty((volume, ALCONSTRAINT_WORDS[self.scalar]), dtype=torch.int32,
+                                       device=self.device))
         words = ALCONSTRAINT_WORDS[self.scalar]
         check(lib().ipc_al_merge(self._ws.handle, 4 * words, self.hash.cell_start.data_ptr(),
                                  self.hash.cell_entries.data_ptr(), int(self.hash.table_size), n_old,

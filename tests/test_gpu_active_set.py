@@ -261,3 +261,28 @@ def test_scan_tile_edges(dev, oracle, T):
     """Bucket counts T + 1 around the scan's tiles of 4096."""
     rng = np.random.default_rng(T)
     check_against_oracle(oracle, dev, random_records(rng, 900, 300, torch.float32), 300, torch.float32, T, 1024)
+
+
+@pytest.mark.parametrize("n_old,n_new", [(0, 0), (0, 3), (3, 0), (300, 700)])
+def test_merge_writes_all_of_uncleared_memory(dev, n_old, n_new):
+    """The destination comes from memory that held something else: its buckets
+    and its tail past the entries are the kernels' own."""
+    rng = np.random.default_rng(n_old + n_new)
+    sets = []
+    for n, base in ((n_old, 0), (n_new, 1 << 20)):
+        if n == 0:
+            sets.append(ActiveSet(1024, dev))
+            continue
+        words = random_records(rng, n, 64, torch.float32, key_base=base)
+        sets.append(gpu_create(dev, words, 64, torch.float32, 128, 1024)[0])
+    A, B = sets
+    counts = A.count(), B.count()
+    junk = [torch.full((s,), -1, dtype=torch.int32, device=dev) for s in (2 * max(1, sum(counts)) + 1,
+                                                                         26 * max(1, sum(counts)))]
+    torch.cuda.synchronize()
+    del junk
+    A.merge(B)
+    start, entries = A.hash.cell_start.cpu().numpy(), A.hash.cell_entries.cpu().numpy()
+    assert start[0] == 0 and (np.diff(start) >= 0).all() and start[-1] == sum(counts)
+    assert A.capacity == max(1, sum(counts)) and not entries[start[-1]:].any()
+    assert len({tuple(k) for k in entries[:start[-1], 4:6]}) == sum(counts)
