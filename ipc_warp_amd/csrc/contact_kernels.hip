@@ -172,11 +172,21 @@ struct ValueStageT<double> {
   float4 out[64 * 9];
 };
 template <typename R>
-struct HessianStageT {
+struct HessianStageT;
+template <>
+struct HessianStageT<float> {
   union {
-    ForceSums<R, 4> force;
-    R f[64 * 12];
-    ValueStageT<R> val;
+    ForceSums<float, 4> force;
+    float f[64 * 12];
+    ValueStageT<float> val;
+  } u[4];
+  int v[4][64 * 4];
+};
+template <>
+struct HessianStageT<double> {
+  union {
+    double f[64 * 12];
+    ValueStageT<double> val;
   } u[4];
   int v[4][64 * 4];
 };
@@ -258,13 +268,19 @@ __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int b
   // twist: 2.8M lines, 0.48M so, and the kernel 237 and 169 us; 600k that share
   // none: 108 and 125). The sparse waves of a short list take the
   // work of a full one for a quarter of the contacts (150k in fp64: 110 us,
-  // 104 without), and add their force components transposed from LDS, value
-  // j by lane j % 64, so that an instruction touches a few lines where
-  // vertices are adjacent.
-  if (lpw == 64) {
-    const int verts[4] = {c.x, c.y, c.z, c.w};
-    add_forces(st.u[wave].force, verts, force, active, b);
-  } else {
+  // 104 without), and the fp64 kernel is bound by its arithmetic (no faster
+  // without any atomic): these add their force components transposed from
+  // LDS, value j by lane j % 64, so that an instruction touches a few lines
+  // where vertices are adjacent.
+  bool summed = false;
+  if constexpr (sizeof(R) == 4) {
+    if (lpw == 64) {
+      const int verts[4] = {c.x, c.y, c.z, c.w};
+      add_forces(st.u[wave].force, verts, force, active, b);
+      summed = true;
+    }
+  }
+  if (!summed) {
     R* sf = st.u[wave].f;
     int* sv = st.v[wave];
     if (lane < lpw) {
