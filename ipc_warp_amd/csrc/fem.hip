@@ -153,6 +153,7 @@ __device__ inline M3 pk1(const M3& F, const Snh& s) {
 struct Tangent {
   M3 F, cof;
   float Ic1, distortional, volumetric;
+  float F0[3], cof0[3];  // 0 times each row of F and cof: zero, or NaN where the row is not finite
 };
 __device__ inline Tangent tangent_of(const M3& F, const Snh& s) {
   Tangent t;
@@ -161,19 +162,27 @@ __device__ inline Tangent tangent_of(const M3& F, const Snh& s) {
   t.Ic1 = ddot(F, F) + 1.0f;
   t.distortional = s.mu * (1.0f - 1.0f / t.Ic1);
   t.volumetric = s.lam * (det3(F) - s.alpha);
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    t.F0[r] = (0.0f * F.m[r][0] + 0.0f * F.m[r][1]) + 0.0f * F.m[r][2];
+    t.cof0[r] = (0.0f * t.cof.m[r][0] + 0.0f * t.cof.m[r][1]) + 0.0f * t.cof.m[r][2];
+  }
   return t;
 }
 
 // Directional derivative of PK1 at F (fem/snh.py:43-84) along a dF whose only
 // nonzero row is row k, g: about half the operations of the dense form, whose
-// other terms add exact zeros. g x b with g = g_c e_k (a column of dF) has
-// components p, q = k + 1, k + 2 (mod 3) only: -g_c b_q and g_c b_p.
+// other terms add exact zeros, or NaN where F or its cofactors have overflowed
+// (their products with zero are kept: F0, cof0). g x b with g = g_c e_k (a
+// column of dF) has components p, q = k + 1, k + 2 (mod 3) only: -g_c b_q and
+// g_c b_p.
 template <int k>
 __device__ inline M3 tangent_row(const Tangent& t, const float g[3], const Snh& s) {
   constexpr int p = (k + 1) % 3, q = (k + 2) % 3;
-  const float dIc = 2.0f * (t.F.m[k][0] * g[0] + t.F.m[k][1] * g[1] + t.F.m[k][2] * g[2]);
+  const float dIc = 2.0f * ((t.F.m[k][0] * g[0] + t.F.m[k][1] * g[1] + t.F.m[k][2] * g[2]) + (t.F0[p] + t.F0[q]));
   const float d_distortional = s.mu * dIc / (t.Ic1 * t.Ic1);
-  const float dJ = t.cof.m[k][0] * g[0] + t.cof.m[k][1] * g[1] + t.cof.m[k][2] * g[2];
+  const float dJ =
+      (t.cof.m[k][0] * g[0] + t.cof.m[k][1] * g[1] + t.cof.m[k][2] * g[2]) + (t.cof0[p] + t.cof0[q]);
   const float lam_dJ = s.lam * dJ;
   const float vz = t.volumetric * 0.0f;  // dcof's row k is zero
   M3 o;

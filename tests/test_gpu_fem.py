@@ -118,3 +118,37 @@ def test_forces_of_crowded_vertices(dev, oracle, V, n):
     # n terms at most a vertex, in any order
     bound = (n + 1) * 2.0 ** -24 * np.abs(np.asarray(f, np.float64)).sum(0).max()
     assert np.abs(b.cpu().numpy() - np.asarray(f, np.float64).sum(0)).max() <= bound
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e9, 1e13, 3e18, 3e19, 1e25, 3e37])
+def test_overflowing_tets_match_oracle(dev, oracle, scale):
+    """Positions up to the largest floats, single infinite and NaN coordinates,
+    and rest shapes that are flat, tiny or huge: every block is the oracle's,
+    and NaN where its dense products with zero are NaN; forces NaN where its
+    are."""
+    rng = np.random.default_rng(3)
+    n = 256
+    xcs = rng.random((n, 4, 3)).astype(np.float32)
+    x = (rng.normal(size=(n, 4, 3)) * scale).astype(np.float32)
+    xcs[:32, 3] = xcs[:32, 0]
+    xcs[32:64, :, 2] = 0
+    xcs[64:96] *= 1e-12
+    xcs[96:128] *= 1e12
+    x[100:140, :, 0] = 0
+    for k, bad in ((140, np.inf), (160, -np.inf), (180, np.nan)):
+        for e in range(k, k + 12):
+            x[e, (e - k) // 3, (e - k) % 3] = bad
+    xcs, x = xcs.reshape(-1, 3), x.reshape(-1, 3)
+    T = np.arange(4 * n, dtype=np.int32).reshape(n, 4)
+    xcs_t, x_t, T_t = (torch.from_numpy(a).to(dev) for a in (xcs, x, T))
+    Bm, W = ops.tet_rest(xcs_t, T_t)
+    rows = torch.empty(16 * n, dtype=torch.int32, device=dev)
+    cols = torch.empty_like(rows)
+    vals = torch.empty((16 * n, 3, 3), dtype=torch.float32, device=dev)
+    b = torch.zeros_like(x_t)
+    ops.tet_hessian(x_t, T_t, Bm, W, MU, LAM, rows, cols, vals, b)
+    rBm, rW = oracle.tet_rest(xcs, T)
+    _, _, rv, rf = oracle.tet_hessian(x, T, rBm, rW, MU, LAM)
+    gv, gf = vals.cpu().numpy(), b.cpu().numpy()
+    assert np.array_equal(np.isnan(gv), np.isnan(rv)) and np.array_equal(np.isnan(gf), np.isnan(rf))
+    assert np.array_equal(gv, rv, equal_nan=True)
