@@ -15,11 +15,11 @@
 // vertex's 6 slots with atomicMin, keeping the smaller key in each slot and
 // carrying the larger one on. Each slot ends with the minimum of the keys that
 // reached it, so the slots hold the 6 smallest keys in order. A slot only
-// ever falls, so a key above what a plain load finds there passes it by
-// without an atomic: most records of a vertex in many contacts are farther
-// than its six nearest and make none. Record ids are
-// 4 * index + vertex position (EE records first, then PT), so the result does
-// not depend on the order in which lanes run.
+// ever falls, so a key above what a relaxed load finds there passes it by
+// without an atomicMin: most records of a vertex in many contacts are farther
+// than its six nearest and make none. Record ids are 4 * index + vertex
+// position (EE records first, then PT), so the result does not depend on the
+// order in which lanes run.
 #include "ipc_device.hpp"
 #include "ipc_kernels.hpp"
 
@@ -42,9 +42,13 @@ __global__ void __launch_bounds__(256) ws_clear_kernel(unsigned long long* __res
 struct Slots {
   unsigned long long k[kWsSlots];
 };
-__device__ __forceinline__ Slots ws_load(const unsigned long long* __restrict__ s) {
+// Relaxed atomic loads: other workgroups lower the slots meanwhile, and only
+// an atomic load promises a whole 64-bit value (a plain copy may be read in
+// any widths).
+__device__ __forceinline__ Slots ws_load(const unsigned long long* s) {
   Slots c;
-  __builtin_memcpy(c.k, s, sizeof(c.k));
+#pragma unroll
+  for (int k = 0; k < kWsSlots; ++k) c.k[k] = __hip_atomic_load(s + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return c;
 }
 // `seen`: values the slots had at some time before.

@@ -112,3 +112,21 @@ def test_features_lane_groups(dev, oracle, n_ee, n_pt, V):
     ref = oracle.warmstart_features(x, None, ee, pt, DHAT)
     got = _gpu(dev, x, None, ee, pt)
     assert np.array_equal(got.view(np.uint32), np.asarray(ref, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("order", ["falling", "rising", "random"])
+def test_features_while_slots_fall(dev, oracle, order):
+    """Many workgroups on three vertices: with falling distances nearly every
+    record lowers slots that others are reading, with rising ones nearly every
+    record passes them by; exact either way."""
+    rng = np.random.default_rng(5)
+    n = 30000
+    d = np.sort(rng.uniform(1e-5, 1e-3, n).astype(np.float32))
+    d = {"falling": d[::-1], "rising": d, "random": rng.permutation(d)}[order]
+    x = np.zeros((3 + n, 3), np.float32)
+    x[:3] = [[-1, 0, -1], [1, 0, -1], [0, 0, 1]]
+    x[3:, 1] = d
+    pt = np.stack([3 + np.arange(n), np.full(n, 0), np.full(n, 1), np.full(n, 2)], 1).astype(np.int32)
+    ee = np.zeros((0, 4), np.int32)
+    ref = oracle.warmstart_features(x, None, ee, pt, DHAT)
+    assert np.array_equal(_gpu(dev, x, None, ee, pt), ref)
