@@ -220,7 +220,7 @@ __device__ inline long long dof_block(const int* poff, const int* pcol, int A, i
   return 16ll * p0 + 4ll * a * len + 4 * lo + c;
 }
 
-__device__ inline float wave_sum(float v) {
+__device__ inline double wave_sum(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
   return v;
@@ -376,10 +376,10 @@ __global__ void finish_values_kernel(const double* acc, long long n, int reps, d
 }
 
 // Forces: vertex i of a free body adds (f, r.x f, r.y f, r.z f) to its
-// body's four rows. A wave walks a run of vertices, a lane adding up while
-// its body stays the same; on a change the wave adds its lanes' terms per
+// body's four rows. A wave walks a run of vertices, a lane adding up in fp64
+// while its body stays the same; on a change the wave adds its lanes' sums per
 // body. (One flush for every 64 vertices made 1844 atomics on each of a
-// body's 12 sums, which serialise: 17 us on 118k vertices, 12 now.)
+// body's 12 sums, which serialise: 26 us on 118k vertices, 13 now.)
 constexpr int kForceRun = 8;
 __global__ __launch_bounds__(kB) void reduce_force_kernel(const float* __restrict__ force,
                                                           const float* __restrict__ rest,
@@ -388,26 +388,26 @@ __global__ __launch_bounds__(kB) void reduce_force_kernel(const float* __restric
   const int lane = threadIdx.x & 63;
   const long long first = (long long)(blockIdx.x * kWaves + (threadIdx.x >> 6)) * 64 * kForceRun + lane;
   int cur = -1;
-  float v[12];
+  double v[12];
 #pragma unroll
-  for (int k = 0; k < 12; ++k) v[k] = 0.0f;
+  for (int k = 0; k < 12; ++k) v[k] = 0.0;
   auto flush = [&]() {
     while (true) {
       const unsigned long long pend = __ballot(cur >= 0);
       if (!pend) break;
       const int B = __shfl(cur, __ffsll(static_cast<long long>(pend)) - 1);
       const bool mine = cur == B;
-      float keep = 0.0f;
+      double keep = 0.0;
 #pragma unroll
       for (int k = 0; k < 12; ++k) {
-        const float s = wave_sum(mine ? v[k] : 0.0f);
+        const double s = wave_sum(mine ? v[k] : 0.0);
         if (lane == k) keep = s;
       }
-      if (lane < 12) atomicAdd(out + 12ll * B + lane, static_cast<double>(keep));
+      if (lane < 12) atomicAdd(out + 12ll * B + lane, keep);
       if (mine) {
         cur = -1;
 #pragma unroll
-        for (int k = 0; k < 12; ++k) v[k] = 0.0f;
+        for (int k = 0; k < 12; ++k) v[k] = 0.0;
       }
     }
   };
@@ -421,12 +421,12 @@ __global__ __launch_bounds__(kB) void reduce_force_kernel(const float* __restric
     if (__ballot(b >= 0 && cur >= 0 && b != cur)) flush();
     if (b >= 0) {
       cur = b;
-      const float f[3] = {force[3 * i], force[3 * i + 1], force[3 * i + 2]};
-      const float c[4] = {1.0f, rest[3 * i], rest[3 * i + 1], rest[3 * i + 2]};
+      const double f[3] = {force[3 * i], force[3 * i + 1], force[3 * i + 2]};
+      const double c[4] = {1.0, rest[3 * i], rest[3 * i + 1], rest[3 * i + 2]};
 #pragma unroll
       for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) v[3 * a + k] = fmaf(c[a], f[k], v[3 * a + k]);
+        for (int k = 0; k < 3; ++k) v[3 * a + k] = fma(c[a], f[k], v[3 * a + k]);
     }
   }
   flush();

@@ -118,3 +118,34 @@ def test_queue_edges_match_oracle(dev, oracle, n, nb):
     err = np.abs(M.values[:nnz].cpu().numpy().astype(np.float64) - v)
     assert (err <= 1e-5 * a + 6e-8 * np.abs(v) + 1e-30).all()
     assert np.abs(rf.cpu().numpy() - rref).max() <= 1e-5 * max(np.abs(rref).max(), 1e-30)
+
+
+def _reduce(dev, nb, body, rest, rows, cols, vals, force):
+    fixed = np.zeros(nb, np.int32)
+    M, rf = AbdReducer().reduce(nb, *(torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+                                      for a in (body, rest, fixed, rows, cols, vals, force)), scale=1.0)
+    torch.cuda.synchronize()
+    return M, rf.cpu().numpy().reshape(-1, 3)
+
+
+@pytest.mark.parametrize("n", [1, 63, 513, 4096, 118000])
+@pytest.mark.parametrize("nb", [1, 3])
+def test_forces_are_summed_in_double(dev, n, nb):
+    """Forces whose sums fp32 partial sums lose (ones beside 2^24, and random
+    ones that nearly cancel): the fp64 sum rounded once to fp32. fp64 sums of n
+    terms, here and in the oracle, are off by n 2^-53 of the magnitudes' sum."""
+    rng = np.random.default_rng(n + nb)
+    body = np.sort(rng.integers(0, nb, n)).astype(np.int32)
+    rest = rng.normal(size=(n, 3)).astype(np.float32)
+    none = np.zeros(1, np.int32)
+    big = np.ones((n, 3), np.float32)
+    big[:: 64 * 3] = 2.0 ** 24
+    for force in (big, rng.normal(size=(n, 3)).astype(np.float32)):
+        _, rf = _reduce(dev, nb, body, rest, none, none, np.zeros((1, 3, 3), np.float32), force)
+        c = np.concatenate([np.ones((n, 1)), rest.astype(np.float64)], 1)
+        t = (c[:, :, None] * force.astype(np.float64)[:, None, :]).reshape(n, 12)
+        want, mag = np.zeros((nb, 12)), np.zeros((nb, 12))
+        np.add.at(want, body, t)
+        np.add.at(mag, body, np.abs(t))
+        err = np.abs(rf.reshape(nb, 12) - want)
+        assert (err <= 2.0 ** -24 * np.abs(want) + 2 * n * 2.0 ** -53 * mag).all()
