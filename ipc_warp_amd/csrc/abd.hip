@@ -16,11 +16,11 @@
 //            BSR: body pair (A, B) owns the 16 blocks (4A + a, 4B + c);
 //   reduce   each workgroup walks a contiguous run of vertex triplets, its
 //            kept ones queued densely in order; its four waves go through
-//            the queue together, wave a summing the blocks (a, 0..3) in fp32
+//            the queue together, wave a summing the blocks (a, 0..3) in fp64
 //            registers while a lane's body pair stays the same; on a change
-//            the wave adds the lanes' sums per body pair (lane order, fp32)
-//            into one of up to 64 fp64 accumulator copies (workgroup index
-//            modulo the copy count) with one atomic per value;
+//            the wave adds the lanes' sums per body pair into one of up to
+//            64 fp64 accumulator copies (workgroup index modulo the copy
+//            count) with one atomic per value;
 //   finish   values = scale * (sum of the copies) rounded to fp32.
 // The forces reduce the same way per vertex (one body per vertex).
 #include <cstdio>
@@ -231,11 +231,13 @@ constexpr int kChunk = 12;  // values per LDS pass of a flush (3 passes of a wav
 
 // Adds every pending lane sum of block row a into the accumulator, one body
 // pair at a time: per pass of kChunk values the lanes of that pair write
-// their sums to LDS (others write zeros), then lane k < kChunk adds value k
-// over the 64 lanes in lane order and issues the fp64 atomic. `out` is this
-// workgroup's accumulator copy.
-__device__ void flush_pairs(int& cur_a, int cur_b, float* acc, int lane, int a, const int* poff, const int* pcol,
-                            float* sh, double* out) {
+// their sums to LDS (others write zeros), then lanes k, 16 + k, 32 + k and
+// 48 + k each add value k over sixteen lanes, the first adds the four and
+// issues the fp64 atomic. (One lane adding all 64 in turn made a list of many
+// body pairs, which flushes every few triplets, wait for those adds.) `out` is
+// this workgroup's accumulator copy.
+__device__ void flush_pairs(int& cur_a, int cur_b, double* acc, int lane, int a, const int* poff, const int* pcol,
+                            double* sh, double* out) {
   while (true) {
     const unsigned long long pend = __ballot(cur_a >= 0);
     if (!pend) break;
@@ -246,20 +248,26 @@ __device__ void flush_pairs(int& cur_a, int cur_b, float* acc, int lane, int a, 
 #pragma unroll
     for (int c = 0; c < 36 / kChunk; ++c) {
 #pragma unroll
-      for (int k = 0; k < kChunk; ++k) sh[k * kPad + lane] = mine ? acc[c * kChunk + k] : 0.0f;
+      for (int i = 0; i < kChunk; ++i) sh[i * kPad + lane] = mine ? acc[c * kChunk + i] : 0.0;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      if (lane < kChunk) {
-        float sum = 0.0f;
-#pragma unroll 16
-        for (int j = 0; j < 64; ++j) sum += sh[lane * kPad + j];
-        atomicAdd(out + 9 * first + c * kChunk + lane, static_cast<double>(sum));  // the four blocks are neighbours
+      const int k = lane & 15, part = lane >> 4;
+      double sum = 0.0;
+      if (k < kChunk) {
+        const double* p = sh + k * kPad + 16 * part;
+        double u[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) u[j & 3] += p[j];
+        sum = (u[0] + u[1]) + (u[2] + u[3]);
       }
+      sum += __shfl_xor(sum, 16);
+      sum += __shfl_xor(sum, 32);
+      if (lane < kChunk) atomicAdd(out + 9 * first + c * kChunk + lane, sum);  // the four blocks are neighbours
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     if (mine) {
       cur_a = -1;
 #pragma unroll
-      for (int k = 0; k < 36; ++k) acc[k] = 0.0f;
+      for (int k = 0; k < 36; ++k) acc[k] = 0.0;
     }
   }
 }
@@ -269,10 +277,12 @@ __device__ void flush_pairs(int& cur_a, int cur_b, float* acc, int lane, int a, 
 // contact list with a fixed body are dropped. With one lane a triplet and all
 // 144 sums in its registers two waves a SIMD did not hide that (289 us for
 // 9.95 million triplets); here the kept ones are first queued, and a wave
-// holds 36 sums, so that five waves a SIMD run (186 us).
+// holds 36 sums, so that four waves a SIMD run. The sums are fp64, since a
+// lane adds up many triplets: fp32 ones lost more the longer the list (and
+// took 58 us instead of 62 for 4 million triplets of two bodies).
 constexpr int kQueuePer = 4;
 constexpr int kQueueTile = kB * kQueuePer;
-__global__ __launch_bounds__(kB) void reduce_hessian_kernel(const int* __restrict__ rows,
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void reduce_hessian_kernel(const int* __restrict__ rows,
                                                             const int* __restrict__ cols,
                                                             const float* __restrict__ vals, int m, int per_block,
                                                             int nv, int nb, const int* __restrict__ body,
@@ -283,7 +293,7 @@ __global__ __launch_bounds__(kB) void reduce_hessian_kernel(const int* __restric
                                                             long long rep_stride) {
   __shared__ int queue[2][kQueueTile];
   __shared__ int num[2][kQueuePer * kWaves];
-  __shared__ float sh[kWaves][kChunk * kPad];
+  __shared__ double sh[kWaves][kChunk * kPad];
   const int lane = threadIdx.x & 63;
   const int a = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave, and its block row
   // workgroups spread their atomics over `reps` copies of the accumulator, so
@@ -291,9 +301,9 @@ __global__ __launch_bounds__(kB) void reduce_hessian_kernel(const int* __restric
   double* out = acc_reps + (blockIdx.x % reps) * rep_stride;
   const long long w0 = (long long)blockIdx.x * per_block;
   const long long w1 = w0 + per_block < m ? w0 + per_block : m;
-  float acc[36];
+  double acc[36];
 #pragma unroll
-  for (int k = 0; k < 36; ++k) acc[k] = 0.0f;
+  for (int k = 0; k < 36; ++k) acc[k] = 0.0;
   int cur_a = -1, cur_b = -1;
   int buf = 0;
   for (long long tile = w0; tile < w1; tile += kQueueTile, buf ^= 1) {
@@ -346,9 +356,9 @@ __global__ __launch_bounds__(kB) void reduce_hessian_kernel(const int* __restric
         cur_b = bj;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
-          const float w = ca * cc[b];
+          const double w = double(ca) * double(cc[b]);
 #pragma unroll
-          for (int k = 0; k < 9; ++k) acc[b * 9 + k] = fmaf(w, h[k], acc[b * 9 + k]);
+          for (int k = 0; k < 9; ++k) acc[b * 9 + k] = fma(w, double(h[k]), acc[b * 9 + k]);
         }
       }
     }

@@ -149,3 +149,25 @@ def test_forces_are_summed_in_double(dev, n, nb):
         np.add.at(mag, body, np.abs(t))
         err = np.abs(rf.reshape(nb, 12) - want)
         assert (err <= 2.0 ** -24 * np.abs(want) + 2 * n * 2.0 ** -53 * mag).all()
+
+
+@pytest.mark.parametrize("n", [1, 63, 1025, 70001, 1000003])
+@pytest.mark.parametrize("nb", [1, 3])
+def test_blocks_are_summed_in_double(dev, oracle, n, nb):
+    """Blocks that a lane adds many of to the same body pair: the fp64 sum
+    rounded once to fp32. fp64 sums of n terms, here and in the oracle, are off
+    by n 2^-53 of the magnitudes' sum, and a term by its two products."""
+    rng = np.random.default_rng(n + nb)
+    nv = 300
+    body = np.sort(rng.integers(0, nb, nv)).astype(np.int32)
+    rest = rng.normal(size=(nv, 3)).astype(np.float32)
+    rows, cols = np.sort(rng.integers(0, nv, (2, n)), axis=1).astype(np.int32)
+    vals = rng.normal(size=(n, 3, 3)).astype(np.float32)
+    vals[:: 64 * 3] = 2.0 ** 24
+    M, _ = _reduce(dev, nb, body, rest, rows, cols, vals, np.zeros((nv, 3), np.float32))
+    o, c, v, a, _ = oracle.abd_reduce(nb, body, rest, np.zeros(nb, np.int32), rows, cols, vals, None, 1.0)
+    nnz = int(o[-1])
+    assert np.array_equal(M.offsets.cpu().numpy(), o)
+    assert np.array_equal(M.columns[:nnz].cpu().numpy(), c)
+    err = np.abs(M.values[:nnz].cpu().numpy().astype(np.float64) - v)
+    assert (err <= 2.0 ** -24 * np.abs(v) + 2 * (n + 4) * 2.0 ** -53 * a).all()
