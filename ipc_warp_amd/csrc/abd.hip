@@ -366,6 +366,19 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void re
   flush_pairs(cur_a, cur_b, acc, lane, a, poff, pcol, sh[a], out);
 }
 
+// Triplets of a workgroup's contiguous run: about 2048 workgroups (twice what
+// the device holds at once), in whole tiles of the queue or, for a list too
+// short for those, whole waves. A list of many body pairs changes pair every
+// few triplets and hands its sums over each time, so a short one has to be
+// spread: 40 bodies, 1600 triplets 264 us with runs of a tile and 23 so
+// (100,000: 85 and 42); two bodies 8.7 and 5.9 (300,000: 12.6 and 14.2).
+long long run_of(long long n) {
+  constexpr long long kWgs = 2048;
+  const long long per = (n + kWgs - 1) / kWgs;
+  const long long unit = per < kQueueTile ? 64 : kQueueTile;
+  return (per + unit - 1) / unit * unit;
+}
+
 // One wave a value, a lane a copy: for few values, whose copies one lane
 // would wait for in turn.
 __global__ void finish_few_kernel(const double* acc, int n, int reps, double scale, float* values) {
@@ -537,8 +550,7 @@ int ipc_abd_reduce_contacts(ipc_abd* w, int n_bodies, const int* body, const flo
   if (blocks == 0) return IPC_OK;
   e = zero_f64(w->acc.as<double>(), 9 * blocks * reps, s);
   if (e == hipSuccess && n_triplets > 0) {
-    // each workgroup a contiguous run of whole tiles, about 2048 workgroups
-    const long long per = ((long long)n_triplets + 2048ll * kQueueTile - 1) / (2048ll * kQueueTile) * kQueueTile;
+    const long long per = run_of(n_triplets);
     hipLaunchKernelGGL(reduce_hessian_kernel, dim3(unsigned((n_triplets + per - 1) / per)), dim3(kB), 0, s, rows, cols,
                        vals, n_triplets, int(per), n_vertices, nb, body, fixed, rest, w->poff.as<int>(),
                        w->pcol.as<int>(), w->acc.as<double>(), int(reps), 9 * blocks);
