@@ -27,29 +27,33 @@ constexpr long long kParams = kOffB4 + kOut;
 static_assert(kParams == IPC_MLP_PARAMS, "parameter layout");
 
 // Phi(z), the normal distribution function, and E = exp(-z^2 / 2):
-//     Phi(-|z|) = E q(|z|),  q(a) = erfcx(a / sqrt 2) / 2 = t P(t),  t = 1 / (1 + 0.3 a)
-// with P of degree 9 fitted for the least relative error on [0, 14] (3.4e-9;
-// beyond it E underflows). About 25 instructions without a branch; erff and
-// expf took four times as many, as long as the matrix products themselves.
-// In fp32 gelu's error is 4.4e-8 rms (erff: 4.9e-8), its derivative's 3.3e-8
-// (2.6e-8), both over normally distributed z; Phi's lower tail keeps its
-// relative precision.
+//     |z| < 1.25:  Phi(z) = 1/2 + z R(z^2)
+//     else:        Phi(-|z|) = E q(|z|),  q(a) = erfcx(a / sqrt 2) / 2 = t P(t),  t = 1 / (1 + 0.3 a)
+// with R and P fitted for the least error of Phi on [0, 1.25] (1.1e-9, as
+// rounded here) and the least relative error of q on [1.25, 14] (2.8e-8;
+// beyond it E underflows). Near zero q changes fast in t, whose rounding alone
+// put 4e-8 into Phi: hence the two ranges. About 30 instructions without a
+// branch; erff and expf took three times as many, as long as the matrix
+// products themselves. In fp32 over normally distributed z gelu's error is
+// 2.1e-8 rms (erff: 2.5e-8), its derivative's 2.5e-8 (2.7e-8). In the lower
+// tail the relative error grows as z^2 (the rounding of E's exponent): 8e-7 at
+// -4, 7e-6 at -13, where 1 + erff has no digit left.
+constexpr float kCentre[7] = {7.110484148e-07f, -1.025638176e-05f, 1.173832643e-04f, -1.189327333e-03f,
+                              9.974518791e-03f, -6.649057567e-02f, 3.989422917e-01f};
+constexpr float kTail[8] = {2.305391431e-02f, -1.159644797e-01f, 1.503848433e-01f, -1.290252805e-02f,
+                            1.113785654e-01f, 1.040908322e-01f,  1.202122197e-01f, 1.196582019e-01f};
 __device__ __forceinline__ float phi_cdf(float z, float& e) {
-  const float a = fabsf(z);
-  e = __builtin_amdgcn_exp2f(z * z * -0.72134752044448170f);
+  const float a = fabsf(z), s = z * z;
+  e = __builtin_amdgcn_exp2f(s * -0.72134752044448170f);
   const float t = __builtin_amdgcn_rcpf(fmaf(0.3f, a, 1.0f));
-  float p = -2.061283588e-02f;
-  p = fmaf(p, t, 1.123758107e-01f);
-  p = fmaf(p, t, -2.280675769e-01f);
-  p = fmaf(p, t, 1.915817857e-01f);
-  p = fmaf(p, t, -7.924740762e-02f);
-  p = fmaf(p, t, 9.605786204e-02f);
-  p = fmaf(p, t, 7.842557132e-02f);
-  p = fmaf(p, t, 1.102273241e-01f);
-  p = fmaf(p, t, 1.195728406e-01f);
-  p = fmaf(p, t, 1.196866333e-01f);
+  float r = kCentre[0], p = kTail[0];
+#pragma unroll
+  for (int k = 1; k < 7; ++k) r = fmaf(r, s, kCentre[k]);
+#pragma unroll
+  for (int k = 1; k < 8; ++k) p = fmaf(p, t, kTail[k]);
   const float lo = e * (p * t);
-  return z >= 0.f ? 1.0f - lo : lo;
+  const float far = z >= 0.f ? 1.0f - lo : lo;
+  return a < 1.25f ? fmaf(z, r, 0.5f) : far;
 }
 __device__ __forceinline__ float gelu(float z) {
   float e;
