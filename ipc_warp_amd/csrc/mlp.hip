@@ -343,23 +343,37 @@ __global__ void __launch_bounds__(kThreads) kFewWaves backward_rows_kernel(const
 
 // The parameter gradients, added into grad, in one launch of three kinds of
 // workgroups: 40 us for 4096 rows, where the eight launches of a VALU product
-// with three row splits (48 workgroups for 256 CUs) took 940 us. Each splits the batch rows, so that the small outputs (147k
-// values) still fill the chip; a split adds its sums with one atomic a value,
-// so there are at most kMaxSplits of them.
+// with three row splits (48 workgroups for 256 CUs) took 940 us. Each splits
+// the batch rows, so that the small outputs (147k values) still fill the chip;
+// a split adds its sums with one fp32 atomic a value, each of which rounds at
+// the size of the whole sum, so there are at most kMaxSplits of them, and
+// kMaxAdders of layer 1, whose splits are its tiles.
 //   [0, b1)        layer 1: dZ1 = (dZ2 W2) * gelu'(Z1) of 64 rows in LDS,
 //                  then dW1 += dZ1^T x and db1
 //   [b1, b1 + b23) layers 3 and 2: a 64 x 128 tile of dW += dZ^T H, its rows
 //                  split over the splits and again over four wave pairs,
 //                  summed in LDS; db from the first column tile's operand
 //   the rest       layer 4: dW4 += dy^T H3, db4
+// A batch of more than kMaxAdders tiles takes layer 1 in a launch of its own
+// after these (b1 = 0): a tile's sums go to memory, over its rows of dZ3, which
+// nothing reads any more, and layer1_sum_kernel adds them up in fp64. Adding
+// every tile's by atomics, 1905 a value for 121,904 rows, put an error of
+// 6.4e-7 into dW1 where dy and x are positive (6e-8 so); the 128 of 8192 rows
+// leave 1.7e-7, less than the 2.7e-7 of the VALU product's chain, and the two
+// launches more cost 40 us there (78 against 117).
 constexpr int kRows1 = 64;
 constexpr int kTileR = 64, kTileC = 128;
 constexpr int kTiles = (kHid / kTileR) * (kHid / kTileC);  // of one layer's dW
 constexpr int kMaxSplits = 16;
+constexpr int kMaxAdders = 128;
+constexpr int kLayer1 = kHid * kIn + kHid;  // dW1 and db1, neighbours in grad
+static_assert(kOffB1 == kOffW1 + kHid * kIn, "dW1 and db1 are neighbours");
 
+// A tile's dW1 and db1: into grad by atomics, or (PART) stored to part.
+template <bool PART>
 __device__ __forceinline__ void layer1_block(float* lds, int block, const float* __restrict__ prm, int n,
                                              const float* __restrict__ x, const float* __restrict__ Z1,
-                                             const float* __restrict__ dz2, float* grad) {
+                                             const float* __restrict__ dz2, float* out) {
   constexpr int RT = kRows1 / 16;
   float* act = lds;
   float* xs = lds + kRows1 * kLd;
@@ -422,12 +436,17 @@ __device__ __forceinline__ void layer1_block(float* lds, int block, const float*
 #pragma unroll
     for (int b = 0; b < 3; ++b)
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        unsafeAtomicAdd(grad + kOffW1 + (c0 + 16 * a + 4 * g + q) * kIn + 16 * b + j, acc[a][b][q]);
+      for (int q = 0; q < 4; ++q) {
+        float* o = out + (c0 + 16 * a + 4 * g + q) * kIn + 16 * b + j;
+        if (PART) *o = acc[a][b][q];
+        else unsafeAtomicAdd(o, acc[a][b][q]);
+      }
   if (threadIdx.x < kHid) {
     float s = 0.f;
     for (int r = 0; r < kRows1; ++r) s += act[r * kLd + threadIdx.x];
-    unsafeAtomicAdd(grad + kOffB1 + threadIdx.x, s);
+    float* o = out + kHid * kIn + threadIdx.x;
+    if (PART) *o = s;
+    else unsafeAtomicAdd(o, s);
   }
 }
 
@@ -519,33 +538,46 @@ __device__ __forceinline__ void dw_tile_block(float* lds, int tile, int k_begin,
 
 __device__ __forceinline__ void layer4_block(float* lds, int k_begin, int k_end, const float* __restrict__ dy,
                                              const float* __restrict__ H3, float* grad) {
+  // fp32 sums of kFold rows, those in fp64: one chain of a split's rows lost
+  // more the larger the batch
+  constexpr int kFold = 32, kParts = kThreads / kHid;
   const int c = threadIdx.x % kHid, part = threadIdx.x / kHid;
-  float s[kOut] = {0.f, 0.f, 0.f}, b[kOut] = {0.f, 0.f, 0.f};
+  double sd[kOut] = {0.0, 0.0, 0.0}, bd[kOut] = {0.0, 0.0, 0.0};
+  for (int r0 = k_begin + part; r0 < k_end; r0 += kFold * kParts) {
+    float s[kOut] = {0.f, 0.f, 0.f}, b[kOut] = {0.f, 0.f, 0.f};
+    const int r1 = min(k_end, r0 + kFold * kParts);
 #pragma unroll 4
-  for (int r = k_begin + part; r < k_end; r += kThreads / kHid) {
-    const float hv = H3[(long long)r * kHid + c];
+    for (int r = r0; r < r1; r += kParts) {
+      const float hv = H3[(long long)r * kHid + c];
+#pragma unroll
+      for (int o = 0; o < kOut; ++o) {
+        const float d = dy[(long long)r * kOut + o];
+        s[o] = fmaf(d, hv, s[o]);
+        b[o] += d;
+      }
+    }
 #pragma unroll
     for (int o = 0; o < kOut; ++o) {
-      const float d = dy[(long long)r * kOut + o];
-      s[o] = fmaf(d, hv, s[o]);
-      b[o] += d;
+      sd[o] += s[o];
+      bd[o] += b[o];
     }
   }
+  double* sums = reinterpret_cast<double*>(lds);
   if (part == 1) {
 #pragma unroll
-    for (int o = 0; o < kOut; ++o) lds[o * kHid + c] = s[o];
+    for (int o = 0; o < kOut; ++o) sums[o * kHid + c] = sd[o];
     if (c == 0) {
 #pragma unroll
-      for (int o = 0; o < kOut; ++o) lds[kOut * kHid + o] = b[o];
+      for (int o = 0; o < kOut; ++o) sums[kOut * kHid + o] = bd[o];
     }
   }
   __syncthreads();
   if (part == 0) {
 #pragma unroll
-    for (int o = 0; o < kOut; ++o) unsafeAtomicAdd(grad + kOffW4 + o * kHid + c, s[o] + lds[o * kHid + c]);
+    for (int o = 0; o < kOut; ++o) unsafeAtomicAdd(grad + kOffW4 + o * kHid + c, float(sd[o] + sums[o * kHid + c]));
     if (c == 0) {
 #pragma unroll
-      for (int o = 0; o < kOut; ++o) unsafeAtomicAdd(grad + kOffB4 + o, b[o] + lds[kOut * kHid + o]);
+      for (int o = 0; o < kOut; ++o) unsafeAtomicAdd(grad + kOffB4 + o, float(bd[o] + sums[kOut * kHid + o]));
     }
   }
 }
@@ -562,7 +594,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
   const long long L = (long long)n * kHid;
   int blk = blockIdx.x;
   if (blk < b1) {
-    layer1_block(lds, blk, prm, n, x, work, dz2, grad);
+    layer1_block<false>(lds, blk, prm, n, x, work, dz2, grad + kOffW1);
     return;
   }
   blk -= b1;
@@ -577,6 +609,31 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
   blk -= b23;
   layer4_block(lds, blk * chunk, min(n, (blk + 1) * chunk), dy, work + 5 * L, grad);
 }
+
+// Layer 1 of a large batch: the sums of the first `parts` tiles over their
+// rows of `part` (dZ3's memory), a last tile of too few rows for that by
+// atomics.
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) layer1_kernel(
+    const float* __restrict__ prm, int n, const float* __restrict__ x, const float* __restrict__ work,
+    const float* __restrict__ dz2, float* part, int parts, float* grad) {
+  __shared__ __align__(16) float lds[kRows1 * (kLd + kLdIn)];
+  const int blk = blockIdx.x;
+  if (blk < parts) layer1_block<true>(lds, blk, prm, n, x, work, dz2, part + (long long)blk * kRows1 * kHid);
+  else layer1_block<false>(lds, blk, prm, n, x, work, dz2, grad + kOffW1);
+}
+
+// grad += the tiles' sums: a lane a value, the tiles split over gridDim.y.
+__global__ void __launch_bounds__(256) layer1_sum_kernel(const float* __restrict__ part, int parts, float* grad) {
+  const int v = blockIdx.x * 256 + threadIdx.x;
+  const int chunk = (parts + gridDim.y - 1) / gridDim.y;
+  const int p0 = blockIdx.y * chunk, p1 = min(parts, p0 + chunk);
+  if (p0 >= p1) return;
+  double s = 0.0;
+#pragma unroll 8
+  for (int p = p0; p < p1; ++p) s += part[(long long)p * kRows1 * kHid + v];
+  unsafeAtomicAdd(grad + kOffW1 + v, float(s));
+}
+static_assert(kLayer1 % 256 == 0, "whole workgroups of values");
 
 // Weighted mean squared error over [n][3]: loss += sum w_i |y_i - t_i|^2 / W,
 // dy = 2 w_i (y_i - t_i) / W with W = sum of weights (passed in).
@@ -660,9 +717,18 @@ hipError_t mlp_backward(const float* prm, int n, const float* x, const float* wo
   if (splits > kMaxSplits) splits = kMaxSplits;
   const int chunk = gblocks(n, splits);
   splits = gblocks(n, chunk);
-  const int b1 = gblocks(n, kRows1), b23 = 2 * kTiles * splits;
+  const int tiles1 = gblocks(n, kRows1), b1 = tiles1 <= kMaxAdders ? tiles1 : 0, b23 = 2 * kTiles * splits;
   hipLaunchKernelGGL(gradients_kernel, dim3(b1 + b23 + splits), dim3(kThreads), 0, s, prm, n, x, work, dy, dz3, dz2,
                      grad, b1, b23, chunk);
+  if (b1 == 0) {
+    // the last tile's rows hold its sums if there are enough of them
+    const int last = n - (tiles1 - 1) * kRows1;
+    const int parts = last * kHid >= kLayer1 ? tiles1 : tiles1 - 1;
+    hipLaunchKernelGGL(layer1_kernel, dim3(tiles1), dim3(kThreads), 0, s, prm, n, x, work, dz2, dz3, parts, grad);
+    const int sums = gblocks(parts, 128);
+    hipLaunchKernelGGL(layer1_sum_kernel, dim3(kLayer1 / 256, sums < kMaxSplits ? sums : kMaxSplits), dim3(256), 0, s,
+                       dz3, parts, grad);
+  }
   return hipGetLastError();
 }
 

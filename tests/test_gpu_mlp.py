@@ -150,3 +150,40 @@ def test_gelu_and_derivative_errors(dev):
     g, d = _gelu_and_derivative(dev, z)
     assert np.array_equal(g[:9], np.array([np.inf, np.nan, np.nan, 0, 0, 1e30, 0, 20, 0], np.float32), equal_nan=True)
     assert np.array_equal(d[:9], np.array([np.nan, np.nan, np.nan, 0.5, 0.5, 1, 0, 1, 0], np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [4096, 8192, 8193, 8240, 8241, 8256, 8257, 32768, 121904])
+def test_large_batch_gradient_sums(dev, n):
+    """Batches around 128 tiles of 64 rows (past them layer 1 is summed in a
+    launch of its own, a last tile of 48 rows and fewer by atomics), and large
+    ones, with positive x and dy so that the sums grow: against fp64 sums of
+    the kept activations. A sum's at most 128 fp32 adders each round by
+    2^-24 / sqrt(3) of the sum so far, rms: in all 2^-24 sqrt(128) / 3 = 2.2e-7,
+    and a tile's own terms 3e-8."""
+    rng = np.random.default_rng(n)
+    net = warmstart.MLP(dev, params=torch.from_numpy(mlp.init(4).astype(np.float32)).to(dev))
+    x = torch.from_numpy(np.abs(rng.standard_normal((n, mlp.IN))).astype(np.float32)).to(dev)
+    dy = torch.from_numpy(np.abs(rng.standard_normal((n, mlp.OUT))).astype(np.float32)).to(dev)
+    _, work = net.forward(x, keep=True)
+    grad = torch.zeros_like(net.params)
+    net.backward(x, work, dy, grad)
+    W, at, o = {}, {}, 0
+    for name, shape in mlp.SHAPES:
+        at[name] = slice(o, o + int(np.prod(shape)))
+        W[name] = net.params[at[name]].double().view(shape)
+        o = at[name].stop
+    Z1, H1, Z2, H2, Z3, H3 = (w.double() for w in work.view(6, n, mlp.HID))
+    D = dy.double()
+
+    def slope(z):
+        return 0.5 * torch.erfc(-z / 2 ** 0.5) + z * torch.exp(-0.5 * z * z) / (2 * np.pi) ** 0.5
+
+    d3 = (D @ W["W4"]) * slope(Z3)
+    d2 = (d3 @ W["W3"]) * slope(Z2)
+    d1 = (d2 @ W["W2"]) * slope(Z1)
+    want = {"W4": D.T @ H3, "b4": D.sum(0), "W3": d3.T @ H2, "b3": d3.sum(0), "W2": d2.T @ H1, "b2": d2.sum(0),
+            "W1": d1.T @ x.double(), "b1": d1.sum(0)}
+    for name, w in want.items():
+        err = float((grad[at[name]].double() - w.reshape(-1)).norm() / w.norm())
+        print(f"{name} {err:.2e}", end=" ", flush=True)
+        assert err <= 2.5e-7, name
