@@ -462,20 +462,65 @@ __global__ __launch_bounds__(kB) void bsr_pattern_kernel(const int* __restrict__
   if (r == nr - 1 && threadIdx.x % kPatternLanes == 0) seg[total] = start[nr];
 }
 
-// Block values: nine lanes a block, one for each value, seven blocks a wave.
-// A block's next nine triplets are read by its lanes together, then their
-// values nine loads at a time, added in ascending triplet order from +0. (One
-// lane a block over values staged in LDS kept 64 lanes waiting for the
-// longest of 64 runs: 153 us on the rod twist's 6.9 million triplets, 130 now.
-// Nine lanes walking nine blocks as one range, so that none waits for a longer
-// one, took 189: the block ends cost more than the waiting.)
+// Block values, a block's triplets added in ascending order from +0. Two ways,
+// by the mean length of the runs (read on the device):
+//   short  a wave takes 64 consecutive blocks, gathers their triplets' values
+//          into LDS a window at a time and adds a block a lane;
+//   long   nine lanes a block, one for each value, seven blocks a wave: a
+//          block's next nine triplets are read by its lanes together, then
+//          their values nine loads at a time.
+// With one lane a block 64 lanes wait for the longest of 64 runs (16 triplets a
+// block: 49 us for 4 million, 30 with nine); nine lanes a block take ten times
+// the instructions for a run of one (142 us for 4 million, 72 with one lane).
+// The two meet at five. (Nine lanes walking nine blocks as one range, so that
+// none waits for a longer one, took 189 us where nine a block take 130: the
+// block ends cost more than the waiting.) Below 2^17 blocks the waves of 64
+// are too few.
 constexpr int kSumBlocks = 7;
+constexpr int kSumWin = 128;          // entries of a window
+constexpr int kSumShort = 5;          // mean run from which nine lanes are faster
+constexpr int kSumFew = 1 << 17;
+
+__device__ __forceinline__ void sum_lane_a_block(int n, const int* __restrict__ seg, const int* __restrict__ tri,
+                                                 const float* __restrict__ vals, float* __restrict__ values, float* s) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (long long o0 = (long long)(blockIdx.x * kWaves + w) * 64; o0 < n; o0 += (long long)gridDim.x * kWaves * 64) {
+    const long long o = o0 + lane;
+    const bool active = o < n;
+    const int mb = active ? seg[o] : 0, me = active ? seg[o + 1] : 0;
+    const int e0 = seg[o0], e1 = seg[o0 + 64 < n ? o0 + 64 : n];
+    float acc[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int w0 = e0; w0 < e1; w0 += kSumWin) {
+      const int cnt = e1 - w0 < kSumWin ? e1 - w0 : kSumWin;
+      for (int k = lane; k < cnt; k += 64) {
+        float v[9];
+        __builtin_memcpy(v, vals + 9ll * tri[w0 + k], sizeof(v));
+#pragma unroll
+        for (int j = 0; j < 9; ++j) s[k * 9 + j] = v[j];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const int lo = mb > w0 ? mb : w0, hi = me < w0 + cnt ? me : w0 + cnt;
+      for (int q = lo; q < hi; ++q) {
+#pragma unroll
+        for (int j = 0; j < 9; ++j) acc[j] += s[(q - w0) * 9 + j];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    if (active) __builtin_memcpy(values + 9 * o, acc, sizeof(acc));
+  }
+}
+
 __global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int* __restrict__ seg,
                                                      const int* __restrict__ tri, const float* __restrict__ vals,
                                                      float* __restrict__ values) {
+  __shared__ float window[kWaves][kSumWin * 9];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane / 9, e = lane - 9 * g;
   const int n = *nnz_p;
+  if (n >= kSumFew && seg[n] < (long long)kSumShort * n) {
+    sum_lane_a_block(n, seg, tri, vals, values, window[w]);
+    return;
+  }
   if (g == kSumBlocks) return;  // the wave's last lane
   for (long long o = (long long)(blockIdx.x * kWaves + w) * kSumBlocks + g; o < n;
        o += (long long)gridDim.x * kWaves * kSumBlocks) {
@@ -503,7 +548,7 @@ __global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int
 
 hipError_t launch_sum(const ipc_bsr* w, int max_blocks, const float* vals, float* values, hipStream_t s) {
   const int need = nblk(max_blocks, kWaves * kSumBlocks);
-  const int g = need < 1 ? 1 : (need < 8192 ? need : 8192);
+  const int g = need < 1 ? 1 : (need < 8192 ? need : 8192);  // strides over the blocks there are
   hipLaunchKernelGGL(bsr_sum_kernel, dim3(g), dim3(kB), 0, s, w->nnz.as<int>(), w->seg.as<int>(), w->slot.as<int>(),
                      vals, values);
   return hipGetLastError();

@@ -267,3 +267,33 @@ def test_row_count_edges(dev, oracle, n_rows):
     vals[rng.random(rows.size) < 0.3] = 0.0
     M = sparse.bsr_from_triplets(n_rows, 50, *_to_dev(dev, rows, cols, vals))
     _same(_host(M), oracle.bsr_from_triplets(n_rows, 50, rows, cols, vals))
+
+
+@pytest.mark.parametrize("blocks", [(1 << 17) - 1, 1 << 17, (1 << 17) + 63])
+@pytest.mark.parametrize("mean", ["short", "under five", "five"])
+def test_sums_by_mean_run(dev, oracle, blocks, mean):
+    """Block counts and mean runs on both sides of the change from nine lanes a
+    block to one, with runs past several windows of 128 entries among short
+    ones and triplets that are dropped; exact against the oracle, and a refill
+    the same."""
+    rng = np.random.default_rng(blocks)
+    runs = rng.integers(1, 3, blocks) if mean == "short" else rng.integers(1, 5, blocks)
+    runs[rng.integers(0, blocks, 40)] = rng.integers(100, 700, 40)
+    if mean != "short":
+        lack = 5 * blocks - runs.sum() - (mean == "under five")
+        runs[rng.permutation(blocks)[:lack // 4]] += 4
+        runs[0] += 5 * blocks - (mean == "under five") - runs.sum()
+    rows, cols = np.arange(blocks) // 11, np.arange(blocks) % 11
+    rows, cols = (np.repeat(a, runs).astype(np.int32) for a in (rows, cols))
+    rows, cols = (np.concatenate([a, np.full(999, 3, np.int32)]) for a in (rows, cols))
+    perm = rng.permutation(rows.size)
+    vals = rng.normal(size=(rows.size, 3, 3)).astype(np.float32)
+    vals[-999:] = 0.0
+    rows, cols, vals = rows[perm], cols[perm], vals[perm]
+    n_rows = int(rows.max()) + 1
+    M = sparse.bsr_from_triplets(n_rows, 11, *_to_dev(dev, rows, cols, vals))
+    ref = oracle.bsr_from_triplets(n_rows, 11, rows, cols, vals)
+    assert int(ref[0][-1]) == blocks
+    _same(_host(M), ref)
+    M.refill(torch.from_numpy(2 * vals).to(dev))
+    _same(_host(M), (ref[0], ref[1], 2 * np.asarray(ref[2])))
