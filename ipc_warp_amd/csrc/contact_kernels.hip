@@ -263,41 +263,20 @@ __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int b
                                   : pair_pt<P, R>(x, c, l0, kappa, true, C, force, nullptr));
   }
   // Forces into b. Device-scope float atomics cost a transaction per cache
-  // line that an instruction touches. A full wave sums its contacts' forces
-  // per vertex first: contacts that lie close share vertices (911k of a rod
-  // twist: 2.8M lines, 0.48M so, and the kernel 237 and 169 us; 600k that share
-  // none: 108 and 125). The sparse waves of a short list take the
-  // work of a full one for a quarter of the contacts (150k in fp64: 110 us,
-  // 104 without), and the fp64 kernel is bound by its arithmetic (no faster
-  // without any atomic): these add their force components transposed from
-  // LDS, value j by lane j % 64, so that an instruction touches a few lines
-  // where vertices are adjacent.
+  // line that an instruction touches. A full wave whose contacts share
+  // vertices with their neighbours sums the forces per vertex first (911k of a
+  // rod twist: 2.8M lines, 0.48M so; the kernel 237 and 169 us). Where nothing
+  // is shared that only costs (600k: 108 and 125 us), and the sparse waves of
+  // a short list take the work of a full one for a quarter of the contacts
+  // (150k in fp64: 110 us, 104 without): these add their forces one by one,
+  // after the values (before them, a shuffled list of 600k took 158 us,
+  // 152 so).
   bool summed = false;
   if constexpr (sizeof(R) == 4) {
-    if (lpw == 64) {
+    if (lpw == 64 && neighbours_share(c, active)) {
       const int verts[4] = {c.x, c.y, c.z, c.w};
       add_forces(st.u[wave].force, verts, force, active, b);
       summed = true;
-    }
-  }
-  if (!summed) {
-    R* sf = st.u[wave].f;
-    int* sv = st.v[wave];
-    if (lane < lpw) {
-#pragma unroll
-      for (int k = 0; k < 12; ++k) sf[lane * 12 + k] = active ? force[k] : R(0);
-      sv[lane * 4 + 0] = c.x;
-      sv[lane * 4 + 1] = c.y;
-      sv[lane * 4 + 2] = c.z;
-      sv[lane * 4 + 3] = c.w;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    for (int j = lane; j < 12 * lpw; j += 64) {
-      const R v = sf[j];
-      if (v != R(0)) {
-        const int slot = j / 12, comp = j - 12 * slot, vert = comp / 3;
-        unsafeAtomicAdd(b + 3 * (long long)sv[slot * 4 + vert] + (comp - 3 * vert), v);
-      }
     }
   }
   if (!active) c = make_int4(0, 0, 0, 0);
@@ -378,6 +357,16 @@ __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int b
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
+  }
+  if (!summed) {
+    // the forces take the values' place
+    R* sf = st.u[wave].f;
+    if (lane < lpw) {
+#pragma unroll
+      for (int k = 0; k < 12; ++k) sf[lane * 12 + k] = active ? force[k] : R(0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    add_forces_one_by_one(sf, sv, lpw, b);
   }
 }
 

@@ -4,9 +4,9 @@
 //
 // The reference launches 16 threads per tet (one per block (i, j)), and
 // each recomputes F, P and the three directional derivatives dP for its
-// column j. Here one lane owns a tet: F and P once, the twelve directional
-// derivatives (j, k) once each, and every block (i, j) column k read from
-// the same dH = -W dP Bm^T. Each value is formed by the reference's own
+// column j. Here two lanes share a tet: F and its cofactors once each, P in
+// the first, six of the twelve directional derivatives (j, k) each, and every
+// block (i, j) column k read from the same dH = -W dP Bm^T. Each value is formed by the reference's own
 // operations in its order, so the blocks equal what its threads compute.
 #include <cstdio>
 
@@ -259,11 +259,12 @@ constexpr int kTetsPerWave = 32;
 constexpr int kTetsPerBlock = 4 * kTetsPerWave;
 
 // Per wave in LDS: its 32 tets' vertex ids and flags; the forces on the way
-// to b, and then one block row (blocks (i, 0..3), 36 floats) of each tet's
+// to b, one by one (f) or summed, and then one block row (blocks (i, 0..3), 36 floats) of each tet's
 // values on the way to memory.
 struct TetStage {
   int v[4][32 * 4];
   int ok[4][32];
+  float f[4][32 * 12];
   union {
     ForceSums<float, 2> force;
     float4 row[32 * 9];
@@ -282,11 +283,12 @@ struct TetStage {
 // row i there), and the wave stores 32 tets' row i with consecutive lanes
 // on consecutive 16-byte words; a lane storing its own tet's 576 bytes
 // touched 64 cache lines per store instruction. Row and column indices go
-// out the same way from the staged vertex ids. The forces are
-// summed per vertex over the wave's 32 tets first (neighbouring tets share
-// vertices, and the device atomics on every corner took 32 of the 131 us of
-// 444,528 tets; 97 with float atomics on a table in LDS, 78 so). Four lanes a tet
-// (95 registers, five waves a SIMD, not 152 and three) took 111: the shared F and
+// out the same way from the staged vertex ids. The forces of tets that share
+// vertices with their neighbours are summed per vertex over the wave's 32
+// first (the device atomics on every corner took 32 of the 131 us of 444,528
+// tets; 97 with float atomics on a table in LDS, 78 so); a list in another
+// order adds them one by one, after the values. Four lanes a tet (95
+// registers, five waves a SIMD, not 162 and three) took 111: the shared F and
 // cofactors weigh more than the waves.
 __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restrict__ x, int nv,
                                                           const int4* __restrict__ T, int n,
@@ -345,18 +347,6 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
       }
     }
   }
-  if (b) {
-    // the second lane of a tet takes over its last two vertices
-    float g[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-      const float u = __shfl(f[6 + q], p, 64);
-      g[q] = half ? u : f[q];
-    }
-    const int verts[2] = {half ? t.z : t.x, half ? t.w : t.y};
-    add_forces(st.u[wave].force, verts, g, ok, b);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the rows take the forces' place
-  }
   int* sv = st.v[wave];
   int* so = st.ok[wave];
   float* sr = reinterpret_cast<float*>(st.u[wave].row);
@@ -367,7 +357,24 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
     sv[p * 4 + 3] = t.w;
     so[p] = ok ? 1 : 0;
   }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  const bool summed = neighbours_share(t, ok && half == 0);
+  if (b) {
+    if (summed) {
+      // the second lane of a tet takes over its last two vertices
+      float g[6];
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        const float u = __shfl(f[6 + q], p, 64);
+        g[q] = half ? u : f[q];
+      }
+      const int verts[2] = {half ? t.z : t.x, half ? t.w : t.y};
+      add_forces(st.u[wave].force, verts, g, ok, b);
+    } else if (half == 0) {
+#pragma unroll
+      for (int q = 0; q < 12; ++q) st.f[wave][p * 12 + q] = f[q];
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the rows take the forces' place
   const long long t0 = (base + first) * 16;
   {
     int4* rows4 = reinterpret_cast<int4*>(rows + t0);
@@ -408,6 +415,7 @@ __global__ void __launch_bounds__(256) tet_hessian_kernel(const float* __restric
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
+  if (b && !summed) add_forces_one_by_one(st.f[wave], sv, nw, b);
 }
 
 // Grid-stride over the tets: each lane sums its tets' energies in double,

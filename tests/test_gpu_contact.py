@@ -239,3 +239,40 @@ def test_long_list_sums_shared_vertices(dev, oracle, kind, distinct):
     f = r_b * times[:, None]
     bound = (TOL + (n / 64 + 64) * 2.0 ** -24) * np.abs(f).max()
     assert np.abs(b.cpu().numpy() - f).max() <= bound
+
+
+@pytest.mark.parametrize("kind", ["pt", "ee"])
+def test_long_list_forces_by_sharing(dev, oracle, kind):
+    """Full waves whose lanes share their vertices with 0 to 63 lanes before
+    (below an eighth of a wave the forces are added one by one, above it
+    summed first: up to 57 contacts of 228 distinct vertices), each wave on
+    vertices of its own, and a last wave of 37. A vertex's force is its pair's
+    times its repetitions, held to that pair's own size: at most 64 equal terms
+    in any order round by 64 2^-24."""
+    n = (1 << 18) + 37
+    x, base = scenes.pair_stream(kind, n, seed=8)
+    i = np.arange(n)
+    share = (i // 64) % 64
+    idx = np.where(i % 64 <= share, i - i % 64, i)
+    xt = torch.from_numpy(x).to(dev)
+    rows = torch.empty(16 * n, dtype=torch.int32, device=dev)
+    cols = torch.empty_like(rows)
+    vals = torch.empty((16 * n, 3, 3), dtype=torch.float32, device=dev)
+    b = torch.zeros_like(xt)
+    ct = torch.from_numpy(base[idx]).to(dev)
+    if kind == "ee":
+        ops.contact_hessian_ee(xt, xt, ct, n, L0, KAPPA, rows, cols, vals, b, 0)
+    else:
+        ops.contact_hessian_pt(xt, ct, n, L0, KAPPA, rows, cols, vals, b, 0)
+    r_rows, r_cols, r_vals, r_b, act = oracle.contact_hessian(kind, x, base, L0, KAPPA, threads=8)
+    it = torch.from_numpy(idx).to(dev)
+    for got, want in ((rows, r_rows), (cols, r_cols)):
+        assert torch.equal(got.view(n, 16), torch.from_numpy(want).to(dev).view(n, 16)[it])
+    want = torch.from_numpy(r_vals.reshape(n, 144)).to(dev)
+    scale = want.abs().amax(1).clamp_min(1e-30)
+    assert (((vals.view(n, 144) - want[it]).abs().amax(1) / scale[it]) <= TOL).all()
+    times = np.bincount(idx, minlength=n).astype(np.float64)
+    f = r_b.reshape(n, 12) * times[:, None]
+    err = np.abs(b.cpu().numpy().reshape(n, 12) - f).max(1)
+    assert (err <= (TOL + 64 * 2.0 ** -24) * np.abs(f).max(1)).all()
+    assert (np.abs(f[times > 0]).max(1) > 0).mean() > 0.9
