@@ -327,8 +327,8 @@ int ipc_ctx_kernel_times(ipc_ctx* ctx, double* total_ms, long long* calls);
 #define IPC_MLP_OUT 3
 #define IPC_MLP_PARAMS 144899
 /* Forward pass. work (float [6 * 256 * n]) keeps Z1, H1, Z2, H2, Z3, H3 for
- * a backward pass; with work = NULL, scratch must be given (float
- * [3 * 256 * n]; the activations stay on the chip and it is left untouched). */
+ * a backward pass; with work = NULL, scratch must not be NULL (it is neither
+ * read nor written: the activations stay on the chip). */
 int ipc_mlp_forward(const float* params, int n, const float* x, float* y, float* work, float* scratch, void* stream);
 /* Inference without a scratch argument: ipc_mlp_forward with work = NULL. No
  * counterpart in the reference: it is for callers that cannot allocate

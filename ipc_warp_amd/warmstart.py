@@ -104,8 +104,8 @@ class MLP:
             check(lib().ipc_mlp_forward(_p(self.params), n, _p(x), _p(y), _p(work), None, stream_handle(self.device)),
                   "mlp_forward")
             return y, work
-        scratch = torch.empty(3 * HID * max(n, 1), dtype=torch.float32, device=self.device)
-        check(lib().ipc_mlp_forward(_p(self.params), n, _p(x), _p(y), None, _p(scratch), stream_handle(self.device)),
+        # the entry point asks for a scratch pointer, and leaves what it points to alone
+        check(lib().ipc_mlp_forward(_p(self.params), n, _p(x), _p(y), None, _p(y), stream_handle(self.device)),
               "mlp_forward")
         return y, None
 

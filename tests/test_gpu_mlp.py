@@ -187,3 +187,14 @@ def test_large_batch_gradient_sums(dev, n):
         err = float((grad[at[name]].double() - w.reshape(-1)).norm() / w.norm())
         print(f"{name} {err:.2e}", end=" ", flush=True)
         assert err <= 2.5e-7, name
+
+
+def test_inference_allocates_its_output_only(dev):
+    net = warmstart.MLP(dev)
+    x = torch.zeros((20000, mlp.IN), device=dev)
+    net.forward(x)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    y, _ = net.forward(x)
+    assert torch.cuda.max_memory_allocated() - before <= y.numel() * 4 + 512
