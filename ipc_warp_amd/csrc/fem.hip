@@ -22,15 +22,6 @@ struct M3 {
   float m[3][3];
 };
 
-__device__ inline M3 mzero() {
-  M3 a;
-#pragma unroll
-  for (int r = 0; r < 3; ++r)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) a.m[r][c] = 0.0f;
-  return a;
-}
-
 __device__ inline M3 from_cols(const float* c0, const float* c1, const float* c2) {
   M3 a;
 #pragma unroll

@@ -3,8 +3,8 @@ dynamic_contacts.py:290-297) against the oracle's restatement.
 
 Bar: offsets, columns and values bit-exact (the kernels sum each block's
 triplets in fp32 in ascending triplet order, as the oracle does), on random
-triplets that reach every row-sort path (rows of <= 64, <= 1024 and more
-entries), on the contact Hessian triplets of the pressed two-cube scene and
+triplets that reach every row-sort path (rows a wave sorts in registers, in a
+workgroup's LDS and in memory), on the contact Hessian triplets of the pressed two-cube scene and
 the screw-and-nut scene, through a pattern refill and through axpy."""
 import ctypes
 
@@ -39,7 +39,7 @@ def _triplets(seed, nr, nc, n):
     rng = np.random.default_rng(seed)
     rows = rng.integers(0, nr, n).astype(np.int32)
     cols = rng.integers(0, nc, n).astype(np.int32)
-    # one row far beyond a wave's LDS sort, one between 64 and 1024 entries
+    # one row far beyond what a wave sorts, one of 700 entries
     rows[: n // 4] = 3
     rows[n // 4: n // 4 + 700] = 11
     rng.shuffle(rows)
@@ -215,7 +215,7 @@ def test_empty_inputs(dev, oracle):
 def test_few_long_rows(dev, oracle):
     """The affine-body pattern the reference assembles (16 body triplets per
     vertex triplet onto a few body rows): 4 rows of ~500k triplets each over
-    32 columns, through the segmented radix sort of long rows."""
+    32 columns, sorted in memory by a workgroup each."""
     import time
 
     rng = np.random.default_rng(9)

@@ -210,7 +210,8 @@ def test_zero_contacts_is_a_noop(dev):
 def test_long_list_sums_shared_vertices(dev, oracle, kind, distinct):
     """Full waves (2^18 contacts and more) whose contacts name few vertices:
     runs of every length in a wave's sorted forces, across its chunks of 64
-    too, and a last wave that is not full."""
+    too. (A single wave's forces are within the rounding of these sums: the
+    next test holds each wave to its own.)"""
     n = (1 << 18) + 37
     x, base = scenes.pair_stream(kind, distinct, seed=distinct)
     idx = np.random.default_rng(distinct).integers(0, distinct, n)

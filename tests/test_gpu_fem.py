@@ -73,9 +73,9 @@ def test_out_of_range_tets_write_zeros(dev):
 @pytest.mark.parametrize("n", [1, 31, 32, 33, 127, 128, 129, 1000])
 def test_partial_workgroups_and_shared_vertices(dev, oracle, n):
     """Tet counts around a wave's 32 and a workgroup's 128, every tet on its
-    own vertices, tets sharing four vertices, and vertices that collide in the
-    workgroup's force table (1024 apart and more): blocks bit-exact, forces
-    within the rounding of the float sums of at most n terms."""
+    own vertices, tets sharing four vertices, and tets 1024 vertices apart and
+    more: blocks bit-exact, forces within the rounding of the float sums of at
+    most n terms."""
     rng = np.random.default_rng(n)
     unit = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]], np.float32)
     for kind in ("own", "shared", "apart"):
@@ -152,3 +152,41 @@ def test_overflowing_tets_match_oracle(dev, oracle, scale):
     gv, gf = vals.cpu().numpy(), b.cpu().numpy()
     assert np.array_equal(np.isnan(gv), np.isnan(rv)) and np.array_equal(np.isnan(gf), np.isnan(rf))
     assert np.array_equal(gv, rv, equal_nan=True)
+
+
+def _slot(v):
+    """The slot of a wave's 256 that vertex v asks for first (two vertices a
+    lane): force_sums.hpp's hash."""
+    h = (v.astype(np.uint64) >> np.uint64(4)) * np.uint64(2654435761) & np.uint64(0xffffffff)
+    return ((h >> np.uint64(12)) & np.uint64(240)) + ((v.astype(np.uint64) + (h >> np.uint64(28))) & np.uint64(15))
+
+
+@pytest.mark.parametrize("slots", [(0,), (5,), (240,), (255,), (0, 15, 16, 240, 255)])
+def test_forces_of_colliding_vertices(dev, oracle, slots):
+    """Strips of tets (each shares a vertex with the one before, so that a wave
+    sums) whose 97 vertices a wave all ask for the same slot of its 256, the
+    first, the last and the last group's among them: every search walks the
+    others' slots, past the last group too. Each vertex is in two tets at
+    most."""
+    rng = np.random.default_rng(slots[0])
+    n = 32 * 5 + 9
+    ids = np.arange(16 * 40000)
+    ids = rng.permutation(ids[np.isin(_slot(ids), slots)])
+    assert ids.size >= 3 * n + 1
+    T = ids[3 * np.arange(n)[:, None] + np.arange(4)].astype(np.int32)
+    nv = int(T.max()) + 1
+    xcs, x = (rng.normal(size=(nv, 3)).astype(np.float32) for _ in range(2))
+    xcs_t, x_t, T_t = (torch.from_numpy(a).to(dev) for a in (xcs, x, T))
+    Bm, W = ops.tet_rest(xcs_t, T_t)
+    rows = torch.empty(16 * n, dtype=torch.int32, device=dev)
+    cols = torch.empty_like(rows)
+    vals = torch.empty((16 * n, 3, 3), dtype=torch.float32, device=dev)
+    b = torch.zeros_like(x_t)
+    ops.tet_hessian(x_t, T_t, Bm, W, MU, LAM, rows, cols, vals, b)
+    rBm, rW = oracle.tet_rest(xcs, T)
+    f = np.zeros((2, nv, 3))
+    for e in range(n):
+        one = oracle.tet_hessian(x[T[e]], np.arange(4, dtype=np.int32)[None], rBm[e:e + 1], rW[e:e + 1], MU, LAM)[3]
+        f[0, T[e]] += one
+        f[1, T[e]] += np.abs(one)
+    assert (np.abs(b.cpu().numpy() - f[0]) <= 3 * 2.0 ** -24 * f[1]).all()

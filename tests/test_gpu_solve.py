@@ -83,10 +83,9 @@ def test_cg_zero_rhs_and_warm_start(dev, system):
     assert it == 0 and res <= goal
 
 
-def test_cg_graph_replays_are_identical(dev, system):
-    """The captured iterations replayed by repeated solves, with eager work
-    and synchronisations between them, give the same bits each time (the
-    sums are in a fixed order) as the first solve."""
+def test_cg_repeated_solves_are_identical(dev, system):
+    """Repeated solves, with other work and synchronisations between them, give
+    the same bits each time (the sums are in a fixed order)."""
     A, ref, V = system
     rng = np.random.default_rng(3)
     b = torch.from_numpy(rng.normal(size=(V, 3)).astype(np.float32)).to(dev)
@@ -96,7 +95,7 @@ def test_cg_graph_replays_are_identical(dev, system):
         it, res, goal = sparse.cg(A, b, x, tol=1e-5, maxiter=2000, jacobi=True)
         torch.cuda.synchronize()
         outs.append((it, res, x.cpu().numpy().copy()))
-        # eager work between replays
+        # other work between the solves
         junk = torch.randn(1 << 20, device=dev).sum()
         sparse.bsr_mv(A, b)
         torch.cuda.synchronize()
