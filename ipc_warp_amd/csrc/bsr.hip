@@ -473,16 +473,17 @@ __global__ __launch_bounds__(kB) void bsr_pattern_kernel(const int* __restrict__
 //   long   nine lanes a block, one for each value, seven blocks a wave: a
 //          block's next nine triplets are read by its lanes together, then
 //          their values nine loads at a time.
-// With one lane a block 64 lanes wait for the longest of 64 runs (16 triplets a
-// block: 49 us for 4 million, 30 with nine); nine lanes a block take ten times
-// the instructions for a run of one (142 us for 4 million, 72 with one lane).
-// The two meet at five. (Nine lanes walking nine blocks as one range, so that
-// none waits for a longer one, took 189 us where nine a block take 130: the
-// block ends cost more than the waiting.) Below 2^17 blocks the waves of 64
-// are too few.
+// With one lane a block 64 lanes wait for the longest of 64 runs (4 million
+// triplets, 16 a block: 49 us, 30 with nine); nine lanes a block take ten times
+// the instructions for a run of one (4 million: 142 us, 69 with one lane), and
+// lose at a mean run of 5.1 still (a tet mesh's 1.44 million blocks: 105 us,
+// 90). At eight they are ahead (34 and 32 us). Below 2^17 blocks the waves of
+// 64 are too few. (Nine lanes walking nine blocks as one range, so that none
+// waits for a longer one, took 189 us where nine a block take 130: the block
+// ends cost more than the waiting.)
 constexpr int kSumBlocks = 7;
 constexpr int kSumWin = 128;          // entries of a window
-constexpr int kSumShort = 5;          // mean run from which nine lanes are faster
+constexpr int kSumShort = 6;          // mean run from which nine lanes take a block
 constexpr int kSumFew = 1 << 17;
 
 __device__ __forceinline__ void sum_lane_a_block(int n, const int* __restrict__ seg, const int* __restrict__ tri,
@@ -514,14 +515,16 @@ __device__ __forceinline__ void sum_lane_a_block(int n, const int* __restrict__ 
   }
 }
 
-__global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int* __restrict__ seg,
+// kept_p: the kept triplets, seg[*nnz_p] too, but read beside the block count
+// instead of after it.
+__global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int* kept_p, const int* __restrict__ seg,
                                                      const int* __restrict__ tri, const float* __restrict__ vals,
                                                      float* __restrict__ values) {
   __shared__ float window[kWaves][kSumWin * 9];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane / 9, e = lane - 9 * g;
-  const int n = *nnz_p;
-  if (n >= kSumFew && seg[n] < (long long)kSumShort * n) {
+  const int n = *nnz_p, kept = *kept_p;
+  if (n >= kSumFew && kept < (long long)kSumShort * n) {
     sum_lane_a_block(n, seg, tri, vals, values, window[w]);
     return;
   }
@@ -550,11 +553,11 @@ __global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int
   }
 }
 
-hipError_t launch_sum(const ipc_bsr* w, int max_blocks, const float* vals, float* values, hipStream_t s) {
+hipError_t launch_sum(const ipc_bsr* w, int n_rows, int max_blocks, const float* vals, float* values, hipStream_t s) {
   const int need = nblk(max_blocks, kWaves * kSumBlocks);
   const int g = need < 1 ? 1 : (need < 8192 ? need : 8192);  // strides over the blocks there are
-  hipLaunchKernelGGL(bsr_sum_kernel, dim3(g), dim3(kB), 0, s, w->nnz.as<int>(), w->seg.as<int>(), w->slot.as<int>(),
-                     vals, values);
+  hipLaunchKernelGGL(bsr_sum_kernel, dim3(g), dim3(kB), 0, s, w->nnz.as<int>(), w->start.as<int>() + n_rows,
+                     w->seg.as<int>(), w->slot.as<int>(), vals, values);
   return hipGetLastError();
 }
 
@@ -717,7 +720,7 @@ int ipc_bsr_from_triplets(ipc_bsr* w, int n_rows, int n_cols, const int* rows, c
       hipLaunchKernelGGL(bsr_pattern_kernel, dim3(nblk(nr, kPatternRows)), dim3(kB), 0, s, start, offsets, nr, bucket,
                          capacity, columns, w->seg.as<int>(), w->nnz.as<int>());
       e = hipGetLastError();
-      if (e == hipSuccess && m > 0) e = launch_sum(w, capacity < m ? capacity : m, vals, values, s);
+      if (e == hipSuccess && m > 0) e = launch_sum(w, nr, capacity < m ? capacity : m, vals, values, s);
     } else {
       e = fill_i32(w->nnz.as<int>(), 1, 0, s);
       if (e == hipSuccess) e = fill_i32(w->seg.as<int>(), 1, 0, s);
@@ -747,7 +750,7 @@ int ipc_bsr_refill(ipc_bsr* w, const float* vals, int n_triplets, float* values,
   if (n_triplets != w->n_triplets) return bsr_fail(IPC_EINVAL, "bsr_refill: triplet count differs from the pattern's");
   if (n_triplets == 0) return IPC_OK;
   if (!vals || !values) return bsr_fail(IPC_EINVAL, "bsr_refill: null pointer");
-  hipError_t e = launch_sum(w, w->max_blocks, vals, values, static_cast<hipStream_t>(stream));
+  hipError_t e = launch_sum(w, w->n_rows, w->max_blocks, vals, values, static_cast<hipStream_t>(stream));
   return bsr_hip(e, "bsr_refill");
 }
 

@@ -270,7 +270,7 @@ def test_row_count_edges(dev, oracle, n_rows):
 
 
 @pytest.mark.parametrize("blocks", [(1 << 17) - 1, 1 << 17, (1 << 17) + 63])
-@pytest.mark.parametrize("mean", ["short", "under five", "five"])
+@pytest.mark.parametrize("mean", ["short", "under six", "six"])
 def test_sums_by_mean_run(dev, oracle, blocks, mean):
     """Block counts and mean runs on both sides of the change from nine lanes a
     block to one, with runs past several windows of 128 entries among short
@@ -280,9 +280,9 @@ def test_sums_by_mean_run(dev, oracle, blocks, mean):
     runs = rng.integers(1, 3, blocks) if mean == "short" else rng.integers(1, 5, blocks)
     runs[rng.integers(0, blocks, 40)] = rng.integers(100, 700, 40)
     if mean != "short":
-        lack = 5 * blocks - runs.sum() - (mean == "under five")
-        runs[rng.permutation(blocks)[:lack // 4]] += 4
-        runs[0] += 5 * blocks - (mean == "under five") - runs.sum()
+        lack = 6 * blocks - runs.sum() - (mean == "under six")
+        runs[rng.permutation(blocks)[:lack // 5]] += 5
+        runs[0] += 6 * blocks - (mean == "under six") - runs.sum()
     rows, cols = np.arange(blocks) // 11, np.arange(blocks) % 11
     rows, cols = (np.repeat(a, runs).astype(np.int32) for a in (rows, cols))
     rows, cols = (np.concatenate([a, np.full(999, 3, np.int32)]) for a in (rows, cols))
