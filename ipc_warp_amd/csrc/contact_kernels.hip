@@ -240,9 +240,9 @@ __device__ __forceinline__ void write_values(const float* sc, float4* so, float*
 // lines with 16 bytes each, and those stores took about half of the kernel's
 // time. Row and column indices are stored from the staged vertex ids. The
 // fp64 values go through LDS in eight passes, each lane expanding half of a
-// block row of its contact (144 bytes) before the wave stores the halves:
-// there the arithmetic is the bound (150k records 102 us, 100 without any
-// store).
+// block row of its contact (144 bytes) before the wave stores the halves: at
+// 16 contacts a wave the stores hide behind the arithmetic (150k records 102
+// us, 100 without any store).
 template <bool EE, typename P, typename R>
 __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int block, HessianStageT<R>& st) {
   const P* __restrict__ x = A.x;
@@ -264,13 +264,12 @@ __device__ __forceinline__ void hessian_block(const HessianArgsT<P, R>& A, int b
   }
   // Forces into b. Device-scope float atomics cost a transaction per cache
   // line that an instruction touches. A full wave whose contacts share
-  // vertices with their neighbours sums the forces per vertex first (911k of a
-  // rod twist: 2.8M lines, 0.48M so; the kernel 237 and 169 us). Where nothing
-  // is shared that only costs (600k: 108 and 125 us), and the sparse waves of
-  // a short list take the work of a full one for a quarter of the contacts
-  // (150k in fp64: 110 us, 104 without): these add their forces one by one,
-  // after the values (before them, a shuffled list of 600k took 158 us,
-  // 152 so).
+  // vertices with their neighbours sums the forces per vertex first (939k of a
+  // rod twist: the kernel 220 us one by one, 171 so). Where nothing is shared
+  // that only costs (600k: 119 and 129 us), and the sparse waves of a short
+  // list take the work of a full one for a quarter of the contacts (150k in
+  // fp64: 110 us, 104 without): these add their forces one by one, after the
+  // values (before them, a shuffled list of 600k took 158 us, 152 so).
   bool summed = false;
   if constexpr (sizeof(R) == 4) {
     if (lpw == 64 && neighbours_share(c, active)) {
@@ -724,8 +723,13 @@ static inline int blocks_for(long long n, int bs) { return int((n + bs - 1) / bs
 // EE and PT halves of one launch share the device, so they are spread by
 // their total length (a PT list of 237k beside 697k EE contacts spread over
 // 16 lanes a wave issued four times the instructions it needed).
+// The lanes are those that were best at 5,000 contacts (PT, us with 16, 32 and
+// 64 lanes: 12.4, 15.6 and 18.7 in fp32, 15.8, 16.3 and 18.4 in fp64), and the
+// line is higher than it should be: from some 20,000 on more lanes are faster
+// (18.0, 15.4, 19.4; 24.6, 18.2, 20.1), at 150,000 by far (66, 43, 41; 92, 55,
+// 53).
 constexpr int kSpreadBelow = 1 << 18;
-constexpr int kSpreadLanes = 16;        // Hessian (measured best of 4..64 at ~5e3 contacts)
+constexpr int kSpreadLanes = 16;        // Hessian
 constexpr int kSpreadLanesEnergy = 32;  // energy (no Hessian, shorter chain)
 static inline int lanes_per_wave(int n, int spread = kSpreadLanes) { return n < kSpreadBelow ? spread : 64; }
 static inline int blocks_spread(int n, int lpw) { return blocks_for(blocks_for(n, lpw), 4); }  // 4 waves per block

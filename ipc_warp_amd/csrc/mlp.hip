@@ -187,9 +187,9 @@ __device__ __forceinline__ void stage_rows(float* dst, int ld, const float* __re
 // All four layers of R rows in one workgroup: the activations stay in LDS and
 // the weights (0.58 MB) come from L2. KEEP stores Z and H of each layer. The
 // bound is the CU's own reads of the weights (64 bytes of each of 16 rows an
-// instruction) beside the products: 20 us for up to 4096 rows, where four
-// launches of a VALU product took 120 us; 89 of 148 TFLOP/s at 121,904 rows
-// (17 before).
+// instruction) beside the products: 23 us for up to 4096 rows, where four
+// launches of a VALU product took 120 us; 84 of 148 TFLOP/s at 121,904 rows
+// (45 before).
 template <int R, bool KEEP>
 __device__ __forceinline__ void layer_out(f4 acc[R / 16][2], float* act, const float bias[2], float* __restrict__ Z,
                                           float* __restrict__ H, long long r0, int n, int c0, int l) {
