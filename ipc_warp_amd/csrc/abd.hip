@@ -228,46 +228,80 @@ __device__ inline double wave_sum(double v) {
 
 constexpr int kPad = 65;    // LDS row pitch of the flush table (conflict-free both ways)
 constexpr int kChunk = 12;  // values per LDS pass of a flush (3 passes of a wave's 36)
+constexpr int kFlushPairs = 64 / kChunk;  // body pairs of a flush's batch
 
-// Adds every pending lane sum of block row a into the accumulator, one body
-// pair at a time: per pass of kChunk values the lanes of that pair write
-// their sums to LDS (others write zeros), then lanes k, 16 + k, 32 + k and
-// 48 + k each add value k over sixteen lanes, the first adds the four and
-// issues the fp64 atomic. (One lane adding all 64 in turn made a list of many
-// body pairs, which flushes every few triplets, wait for those adds.) `out` is
-// this workgroup's accumulator copy.
+// Adds every pending lane sum of block row a into the accumulator, up to
+// kFlushPairs body pairs at a time: per pass of kChunk values every lane writes
+// its sums to LDS, then lane 12 p + k adds value k over the lanes of the batch's
+// pair p and issues the fp64 atomic. A single pair (a list of few bodies) has
+// four lanes a value add sixteen lanes each. A list of many body pairs flushes
+// every few triplets: one pair at a time it waited for LDS (3 million triplets
+// of 1000 bodies 2170 us a call, 770 so). `out` is this workgroup's accumulator
+// copy.
 __device__ void flush_pairs(int& cur_a, int cur_b, double* acc, int lane, int a, const int* poff, const int* pcol,
                             double* sh, double* out) {
   while (true) {
-    const unsigned long long pend = __ballot(cur_a >= 0);
-    if (!pend) break;
-    const int leader = __ffsll(static_cast<long long>(pend)) - 1;
-    const int A = __shfl(cur_a, leader), B = __shfl(cur_b, leader);
-    const bool mine = cur_a == A && cur_b == B;
-    const long long first = dof_block(poff, pcol, A, B, a, 0);
+    // the batch's pairs; lane 12 p + k keeps those of pair p
+    unsigned long long left = __ballot(cur_a >= 0), taken = 0ull, mask = 0ull;
+    if (!left) break;
+    const int mine = lane / kChunk, k = lane - kChunk * mine;
+    int A = -1, B = -1, pairs = 0;
+#pragma unroll 1
+    for (; pairs < kFlushPairs && left; ++pairs) {
+      const int leader = __ffsll(static_cast<long long>(left)) - 1;
+      const int pa = __builtin_amdgcn_readlane(cur_a, leader), pb = __builtin_amdgcn_readlane(cur_b, leader);
+      const unsigned long long m = __ballot(cur_a == pa && cur_b == pb);
+      if (mine == pairs) {
+        A = pa;
+        B = pb;
+        mask = m;
+      }
+      left &= ~m;
+      taken |= m;
+    }
+    const bool add = mine < pairs;
+    double* to = out;
+    if (pairs == 1) to += 9 * dof_block(poff, pcol, __shfl(A, 0), __shfl(B, 0), a, 0);
+    else if (add) to += 9 * dof_block(poff, pcol, A, B, a, 0);
+    const bool in = (taken >> lane) & 1;
 #pragma unroll
     for (int c = 0; c < 36 / kChunk; ++c) {
 #pragma unroll
-      for (int i = 0; i < kChunk; ++i) sh[i * kPad + lane] = mine ? acc[c * kChunk + i] : 0.0;
+      for (int i = 0; i < kChunk; ++i) sh[i * kPad + lane] = in ? acc[c * kChunk + i] : 0.0;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const int k = lane & 15, part = lane >> 4;
-      double sum = 0.0;
-      if (k < kChunk) {
-        const double* p = sh + k * kPad + 16 * part;
-        double u[4] = {0.0, 0.0, 0.0, 0.0};
+      if (pairs == 1) {
+        const int v = lane & 15, part = lane >> 4;
+        double sum = 0.0;
+        if (v < kChunk) {
+          const double* p = sh + v * kPad + 16 * part;
+          double u[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int j = 0; j < 16; ++j) u[j & 3] += p[j];
-        sum = (u[0] + u[1]) + (u[2] + u[3]);
+          for (int j = 0; j < 16; ++j) u[j & 3] += p[j];
+          sum = (u[0] + u[1]) + (u[2] + u[3]);
+        }
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if (lane < kChunk) atomicAdd(to + c * kChunk + lane, sum);  // the four blocks are neighbours
+      } else if (add) {
+        const double* p = sh + k * kPad;
+        double sum = 0.0;
+        for (unsigned long long m = mask; m;) {
+          double u[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            u[j] = m ? p[__ffsll(static_cast<long long>(m)) - 1] : 0.0;
+            m &= m - 1;  // 0 stays 0
+          }
+          sum += (u[0] + u[1]) + (u[2] + u[3]);
+        }
+        atomicAdd(to + c * kChunk + k, sum);
       }
-      sum += __shfl_xor(sum, 16);
-      sum += __shfl_xor(sum, 32);
-      if (lane < kChunk) atomicAdd(out + 9 * first + c * kChunk + lane, sum);  // the four blocks are neighbours
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    if (mine) {
+    if (in) {
       cur_a = -1;
 #pragma unroll
-      for (int k = 0; k < 36; ++k) acc[k] = 0.0;
+      for (int i = 0; i < 36; ++i) acc[i] = 0.0;
     }
   }
 }
@@ -279,7 +313,7 @@ __device__ void flush_pairs(int& cur_a, int cur_b, double* acc, int lane, int a,
 // 9.95 million triplets); here the kept ones are first queued, and a wave
 // holds 36 sums, so that four waves a SIMD run. The sums are fp64, since a
 // lane adds up many triplets: fp32 ones lost more the longer the list (and
-// took 58 us instead of 62 for 4 million triplets of two bodies).
+// took 58 us instead of 65 for 4 million triplets of two bodies).
 constexpr int kQueuePer = 4;
 constexpr int kQueueTile = kB * kQueuePer;
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void reduce_hessian_kernel(const int* __restrict__ rows,
@@ -337,20 +371,23 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void re
       const bool kept = q + lane < total;
       const long long t = kept ? queue[buf][q + lane] : 0;
       int r = 0, c = 0, bi = -1, bj = -1;
-      float h[9], ca = 1.0f, cc[4];
       if (kept) {
         r = rows[t];
         c = cols[t];
-        __builtin_memcpy(h, vals + 9 * t, sizeof(h));
         bi = body[r];
         bj = body[c];
+      }
+      // a lane moving to another body pair first hands its sums to the wave (the
+      // values are read after that: they would not stay in registers across it)
+      if (__ballot(kept && cur_a >= 0 && (bi != cur_a || bj != cur_b)))
+        flush_pairs(cur_a, cur_b, acc, lane, a, poff, pcol, sh[a], out);
+      float h[9], ca = 1.0f, cc[4];
+      if (kept) {
+        __builtin_memcpy(h, vals + 9 * t, sizeof(h));
         if (a > 0) ca = rest[3ll * r + a - 1];
         cc[0] = 1.0f;
         __builtin_memcpy(cc + 1, rest + 3ll * c, 12);
       }
-      // a lane moving to another body pair first hands its sums to the wave
-      if (__ballot(kept && cur_a >= 0 && (bi != cur_a || bj != cur_b)))
-        flush_pairs(cur_a, cur_b, acc, lane, a, poff, pcol, sh[a], out);
       if (kept) {
         cur_a = bi;
         cur_b = bj;
@@ -372,6 +409,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void re
 // few triplets and hands its sums over each time, so a short one has to be
 // spread: 40 bodies, 1600 triplets 264 us with runs of a tile and 23 so
 // (100,000: 85 and 42); two bodies 8.7 and 5.9 (300,000: 12.6 and 14.2).
+// (Flushed a pair at a time; 12, 22, 6 and 15 us now.)
 long long run_of(long long n) {
   constexpr long long kWgs = 2048;
   const long long per = (n + kWgs - 1) / kWgs;

@@ -192,3 +192,30 @@ def test_run_edges_match_oracle(dev, oracle, n):
     assert np.array_equal(M.columns[:nnz].cpu().numpy(), c)
     err = np.abs(M.values[:nnz].cpu().numpy().astype(np.float64) - v)
     assert (err <= 2.0 ** -24 * np.abs(v) + 2 * (n + 4) * 2.0 ** -53 * a).all()
+
+
+@pytest.mark.parametrize("partners", [1, 2, 4, 5, 6, 30])
+def test_flush_batches_match_oracle(dev, oracle, partners):
+    """Waves that hand over one body pair, up to five in a batch and more than
+    five, with lanes that hold nothing among them: contacts of one body with 1
+    to 30 others, in turn and in runs; the bars of the fp64 sums."""
+    rng = np.random.default_rng(partners)
+    nb, per, k = 64, 9, 9000
+    body = np.repeat(np.arange(nb), per).astype(np.int32)
+    nv = nb * per
+    rest = rng.normal(size=(nv, 3)).astype(np.float32)
+    a = np.sort(rng.integers(0, nb, k))
+    b = (a + np.where(np.arange(k) < k // 2, np.arange(k) % partners, rng.integers(0, partners, k))) % nb
+    quads = np.stack([a * per + rng.integers(0, per, k), a * per + rng.integers(0, per, k),
+                      b * per + rng.integers(0, per, k), b * per + rng.integers(0, per, k)], 1).astype(np.int32)
+    rows, cols = np.repeat(quads, 4, 1).reshape(-1), np.tile(quads, (1, 4)).reshape(-1)
+    n = rows.size
+    vals = rng.normal(size=(n, 3, 3)).astype(np.float32)
+    vals[rng.random(n) < 0.4] = 0.0
+    M, _ = _reduce(dev, nb, body, rest, rows, cols, vals, np.zeros((nv, 3), np.float32))
+    o, c, v, s, _ = oracle.abd_reduce(nb, body, rest, np.zeros(nb, np.int32), rows, cols, vals, None, 1.0)
+    nnz = int(o[-1])
+    assert np.array_equal(M.offsets.cpu().numpy(), o)
+    assert np.array_equal(M.columns[:nnz].cpu().numpy(), c)
+    err = np.abs(M.values[:nnz].cpu().numpy().astype(np.float64) - v)
+    assert (err <= 2.0 ** -24 * np.abs(v) + 2 * (n + 4) * 2.0 ** -53 * s).all()
