@@ -516,23 +516,28 @@ __device__ __forceinline__ void sum_lane_a_block(int n, const int* __restrict__ 
 }
 
 // kept_p: the kept triplets, seg[*nnz_p] too, but read beside the block count
-// instead of after it.
-__global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int* kept_p, const int* __restrict__ seg,
+// instead of after it; so are the first run ends, below the most blocks there
+// can be (seg holds max_blocks + 1).
+__global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int* kept_p, int max_blocks,
+                                                     const int* __restrict__ seg,
                                                      const int* __restrict__ tri, const float* __restrict__ vals,
                                                      float* __restrict__ values) {
   __shared__ float window[kWaves][kSumWin * 9];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane / 9, e = lane - 9 * g;
+  long long o = (long long)(blockIdx.x * kWaves + w) * kSumBlocks + g;
+  int q = 0, end = 0;
+  if (o < max_blocks) {
+    q = seg[o];
+    end = seg[o + 1];
+  }
   const int n = *nnz_p, kept = *kept_p;
   if (n >= kSumFew && kept < (long long)kSumShort * n) {
     sum_lane_a_block(n, seg, tri, vals, values, window[w]);
     return;
   }
   if (g == kSumBlocks) return;  // the wave's last lane
-  for (long long o = (long long)(blockIdx.x * kWaves + w) * kSumBlocks + g; o < n;
-       o += (long long)gridDim.x * kWaves * kSumBlocks) {
-    int q = seg[o];
-    const int end = seg[o + 1];
+  while (o < n) {
     float acc = 0.0f;
     int t = q + e < end ? tri[q + e] : 0;
     while (q < end) {
@@ -550,6 +555,11 @@ __global__ __launch_bounds__(kB) void bsr_sum_kernel(const int* nnz_p, const int
       q += 9;
     }
     values[9 * o + e] = acc;
+    o += (long long)gridDim.x * kWaves * kSumBlocks;
+    if (o < n) {
+      q = seg[o];
+      end = seg[o + 1];
+    }
   }
 }
 
@@ -557,7 +567,7 @@ hipError_t launch_sum(const ipc_bsr* w, int n_rows, int max_blocks, const float*
   const int need = nblk(max_blocks, kWaves * kSumBlocks);
   const int g = need < 1 ? 1 : (need < 8192 ? need : 8192);  // strides over the blocks there are
   hipLaunchKernelGGL(bsr_sum_kernel, dim3(g), dim3(kB), 0, s, w->nnz.as<int>(), w->start.as<int>() + n_rows,
-                     w->seg.as<int>(), w->slot.as<int>(), vals, values);
+                     max_blocks, w->seg.as<int>(), w->slot.as<int>(), vals, values);
   return hipGetLastError();
 }
 
