@@ -220,38 +220,32 @@ __device__ inline long long dof_block(const int* poff, const int* pcol, int A, i
   return 16ll * p0 + 4ll * a * len + 4 * lo + c;
 }
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
-
 constexpr int kPad = 65;    // LDS row pitch of the flush table (conflict-free both ways)
 constexpr int kChunk = 12;  // values per LDS pass of a flush (3 passes of a wave's 36)
-constexpr int kFlushPairs = 64 / kChunk;  // body pairs of a flush's batch
+constexpr int kFlushKeys = 64 / kChunk;  // body pairs, or bodies, of a flush's batch
 
-// Adds every pending lane sum of block row a into the accumulator, up to
-// kFlushPairs body pairs at a time: per pass of kChunk values every lane writes
-// its sums to LDS, then lane 12 p + k adds value k over the lanes of the batch's
-// pair p and issues the fp64 atomic. A single pair (a list of few bodies) has
-// four lanes a value add sixteen lanes each. A list of many body pairs flushes
-// every few triplets: one pair at a time it waited for LDS (3 million triplets
-// of 1000 bodies 2170 us a call, 770 so). `out` is this workgroup's accumulator
-// copy.
-__device__ void flush_pairs(int& cur_a, int cur_b, double* acc, int lane, int a, const int* poff, const int* pcol,
-                            double* sh, double* out) {
+// Hands every pending lane sum of a wave over, N values each, up to kFlushKeys
+// keys (body pairs, or bodies) at a time: per pass of kChunk values every lane
+// writes its sums to LDS, then lane 12 p + k adds value k over the lanes of the
+// batch's key p and issues the fp64 atomic, at to(key) + k. A single key (a list
+// of few bodies) has four lanes a value add sixteen lanes each. A list of many
+// body pairs flushes every few triplets: one pair at a time it waited for LDS (3
+// million triplets of 1000 bodies 2170 us a call, 770 so).
+template <int N, typename To>
+__device__ __forceinline__ void flush_sums(int& cur_a, int cur_b, double* acc, int lane, double* sh, To to) {
+  constexpr int kAhead = N == kChunk ? 8 : 4;  // reads in flight; the block sums leave no registers for more
   while (true) {
-    // the batch's pairs; lane 12 p + k keeps those of pair p
+    // the batch's keys; lane 12 p + k keeps key p
     unsigned long long left = __ballot(cur_a >= 0), taken = 0ull, mask = 0ull;
     if (!left) break;
     const int mine = lane / kChunk, k = lane - kChunk * mine;
-    int A = -1, B = -1, pairs = 0;
+    int A = -1, B = -1, keys = 0;
 #pragma unroll 1
-    for (; pairs < kFlushPairs && left; ++pairs) {
+    for (; keys < kFlushKeys && left; ++keys) {
       const int leader = __ffsll(static_cast<long long>(left)) - 1;
       const int pa = __builtin_amdgcn_readlane(cur_a, leader), pb = __builtin_amdgcn_readlane(cur_b, leader);
       const unsigned long long m = __ballot(cur_a == pa && cur_b == pb);
-      if (mine == pairs) {
+      if (mine == keys) {
         A = pa;
         B = pb;
         mask = m;
@@ -259,17 +253,17 @@ __device__ void flush_pairs(int& cur_a, int cur_b, double* acc, int lane, int a,
       left &= ~m;
       taken |= m;
     }
-    const bool add = mine < pairs;
-    double* to = out;
-    if (pairs == 1) to += 9 * dof_block(poff, pcol, __shfl(A, 0), __shfl(B, 0), a, 0);
-    else if (add) to += 9 * dof_block(poff, pcol, A, B, a, 0);
+    const bool add = mine < keys;
+    double* out = nullptr;
+    if (keys == 1) out = to(__shfl(A, 0), __shfl(B, 0));
+    else if (add) out = to(A, B);
     const bool in = (taken >> lane) & 1;
 #pragma unroll
-    for (int c = 0; c < 36 / kChunk; ++c) {
+    for (int c = 0; c < N / kChunk; ++c) {
 #pragma unroll
       for (int i = 0; i < kChunk; ++i) sh[i * kPad + lane] = in ? acc[c * kChunk + i] : 0.0;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      if (pairs == 1) {
+      if (keys == 1) {
         const int v = lane & 15, part = lane >> 4;
         double sum = 0.0;
         if (v < kChunk) {
@@ -281,27 +275,28 @@ __device__ void flush_pairs(int& cur_a, int cur_b, double* acc, int lane, int a,
         }
         sum += __shfl_xor(sum, 16);
         sum += __shfl_xor(sum, 32);
-        if (lane < kChunk) atomicAdd(to + c * kChunk + lane, sum);  // the four blocks are neighbours
+        if (lane < kChunk) atomicAdd(out + c * kChunk + lane, sum);
       } else if (add) {
         const double* p = sh + k * kPad;
         double sum = 0.0;
         for (unsigned long long m = mask; m;) {
-          double u[4];
+          double u[kAhead];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
+          for (int j = 0; j < kAhead; ++j) {
             u[j] = m ? p[__ffsll(static_cast<long long>(m)) - 1] : 0.0;
             m &= m - 1;  // 0 stays 0
           }
-          sum += (u[0] + u[1]) + (u[2] + u[3]);
+#pragma unroll
+          for (int j = 0; j < kAhead; j += 4) sum += (u[j] + u[j + 1]) + (u[j + 2] + u[j + 3]);
         }
-        atomicAdd(to + c * kChunk + k, sum);
+        atomicAdd(out + c * kChunk + k, sum);
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     if (in) {
       cur_a = -1;
 #pragma unroll
-      for (int i = 0; i < 36; ++i) acc[i] = 0.0;
+      for (int i = 0; i < N; ++i) acc[i] = 0.0;
     }
   }
 }
@@ -333,6 +328,8 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void re
   // workgroups spread their atomics over `reps` copies of the accumulator, so
   // a body pair shared by all is not one chain of atomics per value
   double* out = acc_reps + (blockIdx.x % reps) * rep_stride;
+  // the four blocks (a, 0..3) of a body pair are neighbours
+  const auto blocks_of = [&](int A, int B) { return out + 9 * dof_block(poff, pcol, A, B, a, 0); };
   const long long w0 = (long long)blockIdx.x * per_block;
   const long long w1 = w0 + per_block < m ? w0 + per_block : m;
   double acc[36];
@@ -380,7 +377,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void re
       // a lane moving to another body pair first hands its sums to the wave (the
       // values are read after that: they would not stay in registers across it)
       if (__ballot(kept && cur_a >= 0 && (bi != cur_a || bj != cur_b)))
-        flush_pairs(cur_a, cur_b, acc, lane, a, poff, pcol, sh[a], out);
+        flush_sums<36>(cur_a, cur_b, acc, lane, sh[a], blocks_of);
       float h[9], ca = 1.0f, cc[4];
       if (kept) {
         __builtin_memcpy(h, vals + 9 * t, sizeof(h));
@@ -400,7 +397,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void re
       }
     }
   }
-  flush_pairs(cur_a, cur_b, acc, lane, a, poff, pcol, sh[a], out);
+  flush_sums<36>(cur_a, cur_b, acc, lane, sh[a], blocks_of);
 }
 
 // Triplets of a workgroup's contiguous run: about 2048 workgroups (twice what
@@ -437,49 +434,30 @@ __global__ void finish_values_kernel(const double* acc, long long n, int reps, d
 }
 
 // Forces: vertex i of a free body adds (f, r.x f, r.y f, r.z f) to its
-// body's four rows. A wave walks a run of vertices, a lane adding up in fp64
-// while its body stays the same; on a change the wave adds its lanes' sums per
-// body. (One flush for every 64 vertices made 1844 atomics on each of a
-// body's 12 sums, which serialise: 26 us on 118k vertices, 13 now.)
-constexpr int kForceRun = 8;
+// body's four rows. A wave walks 64 `run` vertices, a lane adding up in fp64
+// while its body stays the same; on a change the wave hands its lanes' sums
+// over, body by body.
 __global__ __launch_bounds__(kB) void reduce_force_kernel(const float* __restrict__ force,
                                                           const float* __restrict__ rest,
                                                           const int* __restrict__ body,
-                                                          const int* __restrict__ fixed, int nv, int nb, double* out) {
-  const int lane = threadIdx.x & 63;
-  const long long first = (long long)(blockIdx.x * kWaves + (threadIdx.x >> 6)) * 64 * kForceRun + lane;
+                                                          const int* __restrict__ fixed, int nv, int nb, int run,
+                                                          double* out) {
+  __shared__ double sh[kWaves][kChunk * kPad];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long long first = (long long)(blockIdx.x * kWaves + w) * 64 * run + lane;
   int cur = -1;
-  double v[12];
+  double v[kChunk];
 #pragma unroll
-  for (int k = 0; k < 12; ++k) v[k] = 0.0;
-  auto flush = [&]() {
-    while (true) {
-      const unsigned long long pend = __ballot(cur >= 0);
-      if (!pend) break;
-      const int B = __shfl(cur, __ffsll(static_cast<long long>(pend)) - 1);
-      const bool mine = cur == B;
-      double keep = 0.0;
-#pragma unroll
-      for (int k = 0; k < 12; ++k) {
-        const double s = wave_sum(mine ? v[k] : 0.0);
-        if (lane == k) keep = s;
-      }
-      if (lane < 12) atomicAdd(out + 12ll * B + lane, keep);
-      if (mine) {
-        cur = -1;
-#pragma unroll
-        for (int k = 0; k < 12; ++k) v[k] = 0.0;
-      }
-    }
-  };
-  for (int q = 0; q < kForceRun; ++q) {
+  for (int k = 0; k < kChunk; ++k) v[k] = 0.0;
+  const auto sums_of = [&](int b, int) { return out + 12ll * b; };
+  for (int q = 0; q < run; ++q) {
     const long long i = first + 64 * q;
     int b = -1;
     if (i < nv) {
       b = body[i];
       if (unsigned(b) >= unsigned(nb) || fixed[b]) b = -1;
     }
-    if (__ballot(b >= 0 && cur >= 0 && b != cur)) flush();
+    if (__ballot(b >= 0 && cur >= 0 && b != cur)) flush_sums<kChunk>(cur, 0, v, lane, sh[w], sums_of);
     if (b >= 0) {
       cur = b;
       const double f[3] = {force[3 * i], force[3 * i + 1], force[3 * i + 2]};
@@ -490,7 +468,18 @@ __global__ __launch_bounds__(kB) void reduce_force_kernel(const float* __restric
         for (int k = 0; k < 3; ++k) v[3 * a + k] = fma(c[a], f[k], v[3 * a + k]);
     }
   }
-  flush();
+  flush_sums<kChunk>(cur, 0, v, lane, sh[w], sums_of);
+}
+static_assert(kChunk == 12, "a body's sums are one pass of a flush");
+
+// Runs of 64 vertices of a wave of reduce_force_kernel. Atomics on one address
+// take some 10 ns in turn, and a body's sums take one from each wave: at most
+// some 256 (118k vertices of two bodies, 64 a wave: 26 us, 11 with four runs).
+// Small bodies end a lane's run early: 64 spheres of 42 vertices took 38 us with
+// eight runs a wave, 5 with one.
+int force_run(int nv, int nb) {
+  const long long per = (nv / nb + 64ll * 256 - 1) / (64ll * 256);
+  return int(per < 1 ? 1 : (per > 8 ? 8 : per));
 }
 
 __global__ void finish_force_kernel(const double* acc, int n, float* out) {
@@ -576,8 +565,11 @@ int ipc_abd_reduce_contacts(ipc_abd* w, int n_bodies, const int* body, const flo
   if (force) {
     e = zero_f64(w->facc.as<double>(), 12ll * nb, s);
     if (e == hipSuccess && n_vertices > 0)
-      hipLaunchKernelGGL(reduce_force_kernel, dim3(nblk(n_vertices, kB * kForceRun)), dim3(kB), 0, s, force, rest, body, fixed,
-                         n_vertices, nb, w->facc.as<double>());
+    {
+      const int run = force_run(n_vertices, nb);
+      hipLaunchKernelGGL(reduce_force_kernel, dim3(nblk(n_vertices, kB * run)), dim3(kB), 0, s, force, rest, body,
+                         fixed, n_vertices, nb, run, w->facc.as<double>());
+    }
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess)
       hipLaunchKernelGGL(finish_force_kernel, dim3(nblk(12 * nb, kB)), dim3(kB), 0, s, w->facc.as<double>(), 12 * nb,

@@ -129,11 +129,12 @@ def _reduce(dev, nb, body, rest, rows, cols, vals, force):
 
 
 @pytest.mark.parametrize("n", [1, 63, 513, 4096, 118000])
-@pytest.mark.parametrize("nb", [1, 3])
+@pytest.mark.parametrize("nb", [1, 3, 40, 1000])
 def test_forces_are_summed_in_double(dev, n, nb):
     """Forces whose sums fp32 partial sums lose (ones beside 2^24, and random
-    ones that nearly cancel): the fp64 sum rounded once to fp32. fp64 sums of n
-    terms, here and in the oracle, are off by n 2^-53 of the magnitudes' sum."""
+    ones that nearly cancel), of bodies from one vertex to runs of many waves:
+    the fp64 sum rounded once to fp32. fp64 sums of n terms, here and in the
+    oracle, are off by n 2^-53 of the magnitudes' sum."""
     rng = np.random.default_rng(n + nb)
     body = np.sort(rng.integers(0, nb, n)).astype(np.int32)
     rest = rng.normal(size=(n, 3)).astype(np.float32)
