@@ -493,8 +493,9 @@ int ipc_abd_destroy(ipc_abd* abd);
  * 16 blocks (4A + a, 4B + c), rows sorted by column; offsets int32
  * [4 n_bodies + 1] always written, columns / values when 16 * pairs <=
  * capacity. Blocks are summed in fp64, then scaled and rounded to fp32 (the
- * order across waves is that of the atomics: results agree to fp64 rounding). When force (float [V][3],
- * the vertex force b) is given, _reduce_contact_force's sums are ADDED to
+ * order across waves is that of the atomics: results agree to fp64
+ * rounding). When force (float [V][3], the vertex force b) is given,
+ * _reduce_contact_force's sums are ADDED to
  * reduced_force (float [4 n_bodies][3], unscaled). Synchronises `stream`
  * once (the pattern size). Returns 0, or the block count when it exceeds
  * capacity (nothing else written). n_bodies <= 8192. */
